@@ -70,8 +70,8 @@ def _x(rng, T, H, xdt):
 @pytest.mark.parametrize("xdt", ["bf16", "f32"])
 @pytest.mark.parametrize("with_shared,with_bias", [(True, True), (False, False)])
 def test_moe_exl3_small(dev, T, xdt, with_shared, with_bias):
-    """H = I = 256, 12 experts, top-4: one-row groups (T = 1), two-row groups (T = 2, 5, 16) and
-    16-row groups on the matrix cores (T = 40); the whole layer against oracle.moe.moe_forward."""
+    """H = I = 256, 12 experts, top-4: one-row groups (T = 1) and 16-row groups (T = 2 to 40;
+    at 40 some experts have more rows than one group holds); the whole layer against oracle.moe.moe_forward."""
     H, I, E, k = 256, 256, 12, 4
     rng = np.random.default_rng(T * 7 + len(xdt) + with_shared)
     host = [_expert_tensors(rng, H, I) for _ in range(E)]

@@ -13,8 +13,8 @@
 // W = diag(suh) (H/sqrt(128)) What (H/sqrt(128)) diag(svh) per 128x128 block, H = Sylvester
 // Hadamard-128, so x W = FWHT(FWHT(x * suh)/sqrt(128) What)/sqrt(128) * svh per 128 chunk.
 //
-// Lane decomposition (exl3_slots.inc, generated and checked by gen_exl3_slots.py): 8 lanes share
-// a tile; lane j owns columns j and j+8 (32 values), loads the tile's 16-byte chunk j (stream
+// Lane decomposition of the decode-only kernels (exl3_slots.inc, generated and checked by
+// gen_exl3_slots.py; the fused GEMM's is in exl3_dev.h): 8 lanes share a tile; lane j owns columns j and j+8 (32 values), loads the tile's 16-byte chunk j (stream
 // dwords 4j..4j+3) and takes dword 4j-1 from its neighbour by a shuffle; every window is one or
 // two constant-offset funnel extracts of those 5 dwords. A wave covers 8 consecutive tiles along
 // N (one 128-column Hadamard block) and reads 1 KB of contiguous trellis per step.
@@ -24,20 +24,15 @@
 
 namespace vybdq {
 
-// LDS of the fused GEMM: the x' stage of a split (fp16, duplicated (x, x) pairs for batch <= 2),
-// then for batches of 4..16 one kExl3WtBytes tile per wave. The per-wave partials
-// [4 waves][BP rows][kExl3RedStride floats] reuse the stage after the loop (4 floats of padding
-// per row put the 16-column groups of 4 batch rows on different banks).
-constexpr int kExl3RedStride = 132;
 // one launch (x rotation per workgroup, output rotation by the last split) up to batch 2; at
-// batch 4..16 the per-workgroup rotation of every batch row costs more than the two extra
+// batch 3..16 the per-workgroup rotation of every batch row costs more than the two extra
 // launches (batch 16 measured 39 us with k_exl3_xprep / k_exl3_out, 68 us in one launch)
 __host__ __device__ constexpr bool exl3_fused(int BP) { return BP <= 2; }
-__host__ __device__ constexpr size_t exl3_xs_bytes(int BP, int kbs) {
-  return BP <= 2 ? static_cast<size_t>(BP) * 16 * kbs * 4 : static_cast<size_t>(BP) * (16 * kbs + 8) * 2;
-}
+// LDS of the fused GEMM: batch <= 2 the x' stage of a split (fp16, rows exl3_xstride apart), reused
+// after the loop for the waves' partials [4][batch rows][kExl3RedStride]; larger batches those alone
+__host__ __device__ constexpr int exl3_xstride(int kbs) { return 16 * kbs + 8; }
 static size_t exl3_lds_bytes(int BP, int kbs) {
-  const size_t main = exl3_xs_bytes(BP, kbs) + (BP >= 4 ? static_cast<size_t>(4) * kExl3WtBytes : 0);
+  const size_t main = exl3_fused(BP) ? static_cast<size_t>(BP) * exl3_xstride(kbs) * 2 : 0;
   const size_t red = static_cast<size_t>(4) * BP * kExl3RedStride * 4;
   return main > red ? main : red;
 }
@@ -117,7 +112,12 @@ __global__ void __launch_bounds__(256) k_exl3_dequant(const uint16_t *__restrict
 //    GEMM workgroup itself for its k-range, in LDS; larger batches: by k_exl3_xprep into the
 //    workspace (a workgroup would otherwise rotate BP chunks per wave before its first weight).
 // 2. z[b][n] over the split's k-range = sum x'[b][k] What[k][n]: each wave a quarter of the
-//    k-range on the block's 128 columns, the waves' partials summed in LDS in a fixed order.
+//    k-range on the block's 128 columns (exl3_mma_run: trellis words straight into matrix-core
+//    operands, every batch size), the waves' partials summed in LDS in a fixed order. Bound by the
+//    hash on the VALU (4.0 instructions per weight, 80% of the issue slots while it runs) and, at one row,
+//    by ~8 us per call that do not scale with K (x rotation, arrival, output rotation). K = 5120,
+//    N = 17408: batch 16 23.2 us (29.2 with the decoded words regrouped through LDS, 7.3
+//    instructions per weight), batch 1 20.0 (20.5 with one dot product per weight and lane, 5.0).
 // 3. y[b][n] = svh[n] * FWHT(sum_s z_s[b][.]) / sqrt(128), sums in split order. Batch <= 2: the
 //    last split of a column block to arrive (a per-block arrival counter, reset by that last
 //    arrival so the counters stay zero between calls) does it; larger batches: k_exl3_out.
@@ -129,279 +129,110 @@ __global__ void __launch_bounds__(256) k_exl3_dequant(const uint16_t *__restrict
 
 template <int XDT>
 __global__ void __launch_bounds__(64) k_exl3_xprep(const void *__restrict__ X, const _Float16 *__restrict__ suh,
-                                                   _Float16 *__restrict__ xp, int B, int64_t K) {
+                                                   _Float16 *__restrict__ xp, int64_t K) {
   const int chunk = blockIdx.x, b = blockIdx.y, lane = threadIdx.x;
   const int64_t k0 = 128 * static_cast<int64_t>(chunk) + 2 * lane;
-  float a0 = 0.f, a1 = 0.f;
-  if (b < B) {
-    a0 = load_elem<XDT>(X, b * K + k0) * static_cast<float>(suh[k0]);
-    a1 = load_elem<XDT>(X, b * K + k0 + 1) * static_cast<float>(suh[k0 + 1]);
-  }
+  float a0 = load_elem<XDT>(X, b * K + k0) * static_cast<float>(suh[k0]);
+  float a1 = load_elem<XDT>(X, b * K + k0 + 1) * static_cast<float>(suh[k0 + 1]);
   fwht128_wave(a0, a1);
   xp[b * K + k0] = static_cast<_Float16>(a0 * kRScale);
   xp[b * K + k0 + 1] = static_cast<_Float16>(a1 * kRScale);
 }
 
-template <int BP>
-__global__ void __launch_bounds__(256) k_exl3_gemm(const uint16_t *__restrict__ trellis, const void *__restrict__ X,
-                                                   int xdt, const _Float16 *__restrict__ suh,
-                                                   const _Float16 *__restrict__ svh, void *__restrict__ Y, int ydt,
-                                                   int B, const _Float16 *__restrict__ xp, float *__restrict__ zpart,
-                                                   uint32_t *__restrict__ arrivals, int64_t K, int NB,
-                                                   int kb_per_split) {
+template <bool FUSED>
+__global__ void __launch_bounds__(256, 4) k_exl3_gemm(const uint16_t *__restrict__ trellis, const void *__restrict__ X,
+                                                      int xdt, const _Float16 *__restrict__ suh,
+                                                      const _Float16 *__restrict__ svh, void *__restrict__ Y, int ydt,
+                                                      int B, int BP, const _Float16 *__restrict__ xp,
+                                                      float *__restrict__ zpart, uint32_t *__restrict__ arrivals,
+                                                      int64_t K, int NB, int kb_per_split) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ int is_last;
   const int g = blockIdx.x, s = blockIdx.y, S = gridDim.y;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  const int t = lane >> 3, j = lane & 7;
   const int KB = static_cast<int>(K / 16);
   const int kb_begin = s * kb_per_split;
   const int kb_end = min(kb_begin + kb_per_split, KB);
   const int nkb = kb_end - kb_begin;
-  // Small batches dot the two fp16 halves of each decoded value with (x, x) (one v_dot2 per weight
-  // and batch row: x lo + x hi, the float32 sum the fp16 value rounds), which saves the half add
-  // and the pairing of decoded values; x' is staged duplicated for that. Larger batches round
-  // the value to fp16 once and share it across the batch rows.
-  constexpr bool HALVES = BP <= 2;
-  constexpr bool FUSED = exl3_fused(BP);  // x rotation and output rotation in this launch
-  // Batches of 4..16 multiply on the matrix cores: each wave writes its decoded values of two
-  // k-blocks into its own LDS tile [128 columns][32 k] (column stride kExl3WtStride bytes), then
-  // runs one v_mfma_f32_16x16x32_f16 per 16-column fragment with the x' rows as the A operand
-  // (rows past the batch read as zero). The VALU keeps only the decode.
-  constexpr bool MMA = BP >= 4;
-  // This wave's k-blocks and the first kD of its trellis chunks, loaded before anything else (they
-  // do not depend on x); the loop keeps kD chunks in flight per lane (a register ring).
-  constexpr int kD = 4;
-  const int per_wave = (nkb + 3) / 4;
-  const int w_begin = wave * per_wave;
-  const int w_end = min(w_begin + per_wave, nkb);
-  const int64_t nb = 8 * static_cast<int64_t>(g) + t;
-  auto load_chunk = [&](int kk) {
-    const int kc = kk < w_end ? kk : (w_end > w_begin ? w_end - 1 : 0);  // in range: re-read the last
-    const int64_t tile = static_cast<int64_t>(kb_begin + kc) * NB + nb;
-    return *reinterpret_cast<const u4 *>(trellis + tile * 64 + 8 * j);
-  };
-  // 1. x' rows of this split: [BP][16 * nkb] fp16 (HALVES: u32 pairs (x, x))
-  const int rows = 16 * nkb;
-  // x' row stride of the stage (elements): the matrix-core A reads take 16 batch rows at once,
-  // so their rows are 16 B apart in the banks (a stride of whole 128-B lines would put all 16
-  // reads on the same banks)
-  const int xstride = MMA ? rows + 8 : rows;
-  const int nch = nkb / 8;
-  // Batch <= 2: each wave rotates the 128-chunks cb = wave, wave + 4, ... of x (batch row cb / nch).
-  // The raw x and suh elements of its first kXP chunks are read before the trellis ring: loads
-  // return in order, so the rotation then waits for these alone, not for the ring behind them.
-  constexpr int kXP = 2;
-  // (x elements k, k + 1 of the chunk's batch row: two f32 words, or one word of two 16-bit
-  // halves; suh k, k + 1 as one word of halves. Kept raw: converting them here would wait.)
-  auto x_raw = [&](int cb, uint32_t (&xv)[2], uint32_t &sv) {
-    const int b = cb / nch, c = cb - b * nch;
-    const int64_t k = 16 * static_cast<int64_t>(kb_begin) + 128 * c + 2 * lane;
-    const int64_t i = static_cast<int64_t>(b < B ? b : 0) * K + k;
-    if (xdt == VYBDQ_F32) __builtin_memcpy(xv, static_cast<const float *>(X) + i, 8);
-    else __builtin_memcpy(xv, static_cast<const uint16_t *>(X) + i, 4);
-    __builtin_memcpy(&sv, suh + k, 4);
-  };
-  uint32_t xw[kXP][2], sw[kXP];
+  // this wave's 64-k steps of the split
+  const int nst = nkb / kExl3Step;
+  const int st0 = nst * wave / 4, st1 = nst * (wave + 1) / 4;
+  const int kb0 = kb_begin + kExl3Step * st0;
+  const int64_t kstride = static_cast<int64_t>(NB) * 64;
+  const uint16_t *base = trellis + kb0 * kstride + 512 * static_cast<int64_t>(g);
+  const int am = lane & 15;
+  f4 acc[8];
+#pragma unroll
+  for (int f = 0; f < 8; ++f) acc[f] = f4{0.f, 0.f, 0.f, 0.f};
   if constexpr (FUSED) {
-#pragma unroll
-    for (int it = 0; it < kXP; ++it)
-      if (wave + 4 * it < BP * nch) x_raw(wave + 4 * it, xw[it], sw[it]);
-  }
-  // Batch > 2: the rotated x' rows are copied from the workspace in 16-byte chunks, four per
-  // thread at a time; the first four are read before the trellis ring for the same reason.
-  const int nc = BP * rows / 8;
-  auto xp_chunk = [&](int i) {
-    const int b = i / (rows / 8), c = i % (rows / 8);
-    return *reinterpret_cast<const u4 *>(xp + b * K + 16 * static_cast<int64_t>(kb_begin) + 8 * c);
-  };
-  auto xs_store = [&](int i, const u4 v) {
-    const int b = i / (rows / 8), c = i % (rows / 8);
-    *reinterpret_cast<u4 *>(reinterpret_cast<_Float16 *>(smem) + b * xstride + 8 * c) = v;
-  };
-  u4 xv4[4];
-  if constexpr (!FUSED) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int i = threadIdx.x + u * blockDim.x;
-      if (i < nc) xv4[u] = xp_chunk(i);
-    }
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  u4 ring[kD];
-#pragma unroll
-  for (int d = 0; d < kD; ++d) ring[d] = load_chunk(w_begin + d);
-  if constexpr (!FUSED) {
-    for (int i0 = threadIdx.x;;) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (i0 + u * blockDim.x < nc) xs_store(i0 + u * blockDim.x, xv4[u]);
-      i0 += 4 * blockDim.x;
-      if (i0 >= nc) break;
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (i0 + u * blockDim.x < nc) xv4[u] = xp_chunk(i0 + u * blockDim.x);
-    }
-  }
-  auto rotate = [&](int cb, const uint32_t (&xv)[2], uint32_t sv) {  // one 128-chunk, whole wave
-    const int b = cb / nch, c = cb - b * nch;
-    const int r = 128 * c + 2 * lane;
-    float a0 = 0.f, a1 = 0.f;
-    if (b < B) {
+    // 1. x' rows of this split: [B][16 nkb] fp16 in LDS; wave w rotates the 128-chunks w, w + 4, ...
+    // of all rows (batch row cb / nch). The raw x and suh words of its first kXP chunks are read before the
+    // trellis ring: loads return in order, so the rotation waits for these alone. (x elements k,
+    // k + 1: two f32 words, or one word of two 16-bit halves; suh likewise. Kept raw: converting them
+    // here would wait.)
+    constexpr int kXP = 2;
+    _Float16 *xs = reinterpret_cast<_Float16 *>(smem);
+    const int xst = exl3_xstride(kb_per_split), nch = nkb / 8, ntask = B * nch;
+    auto x_raw = [&](int cb, uint32_t (&xv)[2], uint32_t &sv) {
+      const int b = cb / nch, c = cb - b * nch;
+      const int64_t k = 16 * static_cast<int64_t>(kb_begin) + 128 * c + 2 * lane, i = static_cast<int64_t>(b) * K + k;
+      if (xdt == VYBDQ_F32) __builtin_memcpy(xv, static_cast<const float *>(X) + i, 8);
+      else __builtin_memcpy(xv, static_cast<const uint16_t *>(X) + i, 4);
+      __builtin_memcpy(&sv, suh + k, 4);
+    };
+    auto rotate = [&](int cb, const uint32_t (&xv)[2], uint32_t sv) {  // one 128-chunk, whole wave
+      const int b = cb / nch, c = cb - b * nch;
+      float a0, a1;
       if (xdt == VYBDQ_F32) { a0 = __uint_as_float(xv[0]); a1 = __uint_as_float(xv[1]); }
       else if (xdt == VYBDQ_F16) { a0 = half_bits_to_f32(xv[0] & 0xffffu); a1 = half_bits_to_f32(xv[0] >> 16); }
       else { a0 = __uint_as_float(xv[0] << 16); a1 = __uint_as_float(xv[0] & 0xffff0000u); }
       a0 *= half_bits_to_f32(sv & 0xffffu);
       a1 *= half_bits_to_f32(sv >> 16);
-    }
-    fwht128_wave(a0, a1);
-    const uint32_t h0 = __builtin_bit_cast(uint16_t, static_cast<_Float16>(a0 * kRScale));
-    const uint32_t h1 = __builtin_bit_cast(uint16_t, static_cast<_Float16>(a1 * kRScale));
-    if constexpr (HALVES) {
-      *reinterpret_cast<u2 *>(reinterpret_cast<uint32_t *>(smem) + b * rows + r) = u2{h0 | (h0 << 16), h1 | (h1 << 16)};
-    } else {
-      *reinterpret_cast<uint32_t *>(reinterpret_cast<_Float16 *>(smem) + b * rows + r) = h0 | (h1 << 16);
-    }
-  };
-  if constexpr (FUSED) {
+      fwht128_wave(a0, a1);
+      *reinterpret_cast<h2 *>(xs + b * xst + 128 * c + 2 * lane) =
+          h2{static_cast<_Float16>(a0 * kRScale), static_cast<_Float16>(a1 * kRScale)};
+    };
+    uint32_t xw[kXP][2], sw[kXP];
 #pragma unroll
     for (int it = 0; it < kXP; ++it)
-      if (wave + 4 * it < BP * nch) rotate(wave + 4 * it, xw[it], sw[it]);
-    for (int cb = wave + 4 * kXP; cb < BP * nch; cb += 4) {
-      uint32_t xv[2], sv;
-      x_raw(cb, xv, sv);
-      rotate(cb, xv, sv);
-    }
-  }
-  __syncthreads();
-  const _Float16 *xs = reinterpret_cast<const _Float16 *>(smem);
-
-  // 2. this split's partial
-  float acc[BP][2];
+      if (wave + 4 * it < ntask) x_raw(wave + 4 * it, xw[it], sw[it]);
+    __builtin_amdgcn_sched_barrier(0);
+    const _Float16 *arow = xs + (am < B ? am : 0) * xst + 16 * (kb0 - kb_begin + (lane >> 4));
+    exl3_mma_run<false>(base, kstride, st1 - st0,
+                 [&] {
 #pragma unroll
-  for (int b = 0; b < BP; ++b) acc[b][0] = acc[b][1] = 0.f;
-  f4 accm[MMA ? 8 : 1];
-#pragma unroll
-  for (int f = 0; f < (MMA ? 8 : 1); ++f) accm[f] = f4{0.f, 0.f, 0.f, 0.f};
-  char *wt = smem + exl3_xs_bytes(BP, kb_per_split) + static_cast<size_t>(wave) * kExl3WtBytes;
-  auto step = [&](int kk, const u4 c) {
-    uint32_t w[6];
-    chunk_window(c, w);
-    if constexpr (HALVES) {
-      // the 16 (x, x) pairs of this k-block per batch row: four 16-B LDS reads
-      uint32_t xq[BP][16];
-#pragma unroll
-      for (int b = 0; b < BP; ++b) {
-        const u4 *src = reinterpret_cast<const u4 *>(reinterpret_cast<const uint32_t *>(smem) + b * rows + 16 * kk);
-#pragma unroll
-        for (int c4 = 0; c4 < 4; ++c4) {
-          const u4 v4 = src[c4];
-          xq[b][4 * c4 + 0] = v4[0];
-          xq[b][4 * c4 + 1] = v4[1];
-          xq[b][4 * c4 + 2] = v4[2];
-          xq[b][4 * c4 + 3] = v4[3];
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < 32; ++q) {
-        const h2 y = __builtin_bit_cast(h2, slot_halves(w, q));
-#pragma unroll
-        for (int b = 0; b < BP; ++b)
-          acc[b][q >> 4] = __builtin_amdgcn_fdot2(y, __builtin_bit_cast(h2, xq[b][q & 15]), acc[b][q >> 4], false);
-      }
-      return;
-    }
-    if constexpr (MMA) {
-      // The 32 slot words of this k-block as they are: word q holds the two fp16 halves of value q
-      // (their sum is the value), q < 16 column c0 at k = 16 kk + q, q >= 16 column c0 + 8. Column
-      // c's 16 words in k order make the tile row [c][k' = 2 k + h], and the MFMA with each x'
-      // value twice in A adds x lo + x hi in float32: no fp16 add or packing of decoded values.
-      const int c0 = 16 * t + j;
-      uint32_t hw[32];
-#pragma unroll
-      for (int q = 0; q < 32; ++q) hw[q] = slot_halves(w, q);
-      u4 *d0 = reinterpret_cast<u4 *>(wt + c0 * kExl3WtStride);
-      u4 *d1 = reinterpret_cast<u4 *>(wt + (c0 + 8) * kExl3WtStride);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        d0[i] = u4{hw[4 * i], hw[4 * i + 1], hw[4 * i + 2], hw[4 * i + 3]};
-        d1[i] = u4{hw[16 + 4 * i], hw[16 + 4 * i + 1], hw[16 + 4 * i + 2], hw[16 + 4 * i + 3]};
-      }
-      // A = x'[m][16 kk + 4 g .. + 4], each value twice (k' = 8 g .. + 8); B = the tile
-      const int m = lane & 15, gk = lane >> 4;
-      u2 xv = u2{0u, 0u};
-      if (m < BP) xv = *reinterpret_cast<const u2 *>(xs + m * xstride + 16 * kk + 4 * gk);
-      const h8 a = __builtin_bit_cast(h8, u4{__builtin_amdgcn_perm(xv[0], xv[0], 0x01000100u),
-                                             __builtin_amdgcn_perm(xv[0], xv[0], 0x03020302u),
-                                             __builtin_amdgcn_perm(xv[1], xv[1], 0x01000100u),
-                                             __builtin_amdgcn_perm(xv[1], xv[1], 0x03020302u)});
-#pragma unroll
-      for (int f = 0; f < 8; ++f) {
-        const h8 b = *reinterpret_cast<const h8 *>(wt + (16 * f + m) * kExl3WtStride + 16 * gk);
-        accm[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, accm[f], 0, 0, 0);
-      }
-      return;
-    }
-    _Float16 v[32];
-    lane_decode(w, v);
-    h2 pj[8], pj8[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      pj[i] = h2{v[2 * i], v[2 * i + 1]};
-      pj8[i] = h2{v[16 + 2 * i], v[16 + 2 * i + 1]};
-    }
-#pragma unroll
-    for (int b = 0; b < BP; ++b) {
-      const u4 *xr = reinterpret_cast<const u4 *>(xs + b * rows + 16 * kk);
-      const u4 x0 = xr[0], x1 = xr[1];
-      const uint32_t xw[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const h2 xv = __builtin_bit_cast(h2, xw[i]);
-        acc[b][0] = __builtin_amdgcn_fdot2(pj[i], xv, acc[b][0], false);
-        acc[b][1] = __builtin_amdgcn_fdot2(pj8[i], xv, acc[b][1], false);
-      }
-    }
-  };
-  // Whole groups of kD k-blocks without conditions, each ring slot refilled right after the step
-  // that consumed it (into the same registers): the loads stay in flight across groups. (A
-  // per-block bound made every slot a merge of two paths, and a refill issued before the step
-  // needed a second register set that was copied back at the loop end; both made the compiler
-  // wait for every load once per group.) The last (fewer than kD) blocks are already in the ring.
-  int k0 = w_begin;
-  for (; k0 + kD <= w_end; k0 += kD) {
-#pragma unroll
-    for (int d = 0; d < kD; ++d) {
-      step(k0 + d, ring[d]);
-      ring[d] = load_chunk(k0 + d + kD);
-      // keeps the refill here: sunk to the end of the group it would leave no load in flight
-      // while the group's last step waits for its own
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-#pragma unroll
-  for (int d = 0; d < kD - 1; ++d)
-    if (k0 + d < w_end) step(k0 + d, ring[d]);
-  // reduce the 4 waves (same columns, different k) in a fixed order
-  __syncthreads();
-  float *red = reinterpret_cast<float *>(smem);  // [4][BP][kExl3RedStride]
-  if constexpr (MMA) {
-    // accm[f][r] = z[batch 4 (lane >> 4) + r][column 16 f + (lane & 15)]
-#pragma unroll
-    for (int f = 0; f < 8; ++f)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int b = 4 * (lane >> 4) + r;
-        if (b < BP) red[(wave * BP + b) * kExl3RedStride + 16 * f + (lane & 15)] = accm[f][r];
-      }
+                   for (int it = 0; it < kXP; ++it)
+                     if (wave + 4 * it < ntask) rotate(wave + 4 * it, xw[it], sw[it]);
+                   for (int cb = wave + 4 * kXP; cb < ntask; cb += 4) {
+                     uint32_t xv[2], sv;
+                     x_raw(cb, xv, sv);
+                     rotate(cb, xv, sv);
+                   }
+                   exl3_barrier();
+                 },
+                 [&](int st, u4 (&v)[2]) {
+                   const u4 *x = reinterpret_cast<const u4 *>(arow + 16 * kExl3Step * st);
+                   v[0] = x[0];
+                   v[1] = x[1];
+                 },
+                 acc);
+    __syncthreads();  // the partials reuse the stage
   } else {
-    const int c0 = 16 * t + j;  // this lane's columns: c0 and c0 + 8
-#pragma unroll
-    for (int b = 0; b < BP; ++b) {
-      red[(wave * BP + b) * kExl3RedStride + c0] = acc[b][0];
-      red[(wave * BP + b) * kExl3RedStride + c0 + 8] = acc[b][1];
-    }
+    const _Float16 *arow = xp + (am < B ? am : 0) * K + 16 * static_cast<int64_t>(kb0 + (lane >> 4));
+    exl3_mma_run<true>(base, kstride, st1 - st0,
+                 [] {},
+                 [&](int st, u4 (&v)[2]) {
+                   const u4 *x = reinterpret_cast<const u4 *>(arow + 16 * kExl3Step * st);
+                   v[0] = x[0];
+                   v[1] = x[1];
+                 },
+                 acc);
   }
+
+  // 2. this split's partial: the 4 waves (same columns, different k) summed in a fixed order
+  float *red = reinterpret_cast<float *>(smem);  // [4][BP][kExl3RedStride]
+  const int wst = BP * kExl3RedStride;
+  exl3_mma_store(acc, red + wave * wst, B);
   __syncthreads();
   const int64_t N = static_cast<int64_t>(NB) * 16;
   auto zp = [&](int split, int b, int c) {
@@ -409,8 +240,8 @@ __global__ void __launch_bounds__(256) k_exl3_gemm(const uint16_t *__restrict__ 
   };
   for (int i = threadIdx.x; i < B * 128; i += blockDim.x) {
     const int b = i / 128, c = i % 128;
-    const float z = ((red[(0 * BP + b) * kExl3RedStride + c] + red[(1 * BP + b) * kExl3RedStride + c]) +
-                     red[(2 * BP + b) * kExl3RedStride + c]) + red[(3 * BP + b) * kExl3RedStride + c];
+    const float *o = red + b * kExl3RedStride + c;
+    const float z = ((o[0] + o[wst]) + o[2 * wst]) + o[3 * wst];
     if constexpr (FUSED) __hip_atomic_store(zp(s, b, c), __float_as_uint(z), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else *zp(s, b, c) = __float_as_uint(z);
   }
@@ -426,32 +257,32 @@ __global__ void __launch_bounds__(256) k_exl3_gemm(const uint16_t *__restrict__ 
   }
   __syncthreads();
   if (!is_last) return;
-  for (int b = wave; b < B; b += 4) {
-    // the splits' partials (this lane's two columns as one 8-byte word) in groups of 8 independent
-    // loads, one round trip per group, added in split order
-    float a0 = 0.f, a1 = 0.f;
-    for (int s0 = 0; s0 < S; s0 += 8) {
-      uint64_t v[8];
+  const int b = wave;  // batch <= 2: one row per wave
+  if (b >= B) return;
+  // the splits' partials (this lane's two columns as one 8-byte word) in groups of 8 independent
+  // loads, one round trip per group, added in split order
+  float a0 = 0.f, a1 = 0.f;
+  for (int s0 = 0; s0 < S; s0 += 8) {
+    uint64_t v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (s0 + u < S)
-          v[u] = __hip_atomic_load(reinterpret_cast<uint64_t *>(zp(s0 + u, b, 2 * lane)), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
+    for (int u = 0; u < 8; ++u)
+      if (s0 + u < S)
+        v[u] = __hip_atomic_load(reinterpret_cast<uint64_t *>(zp(s0 + u, b, 2 * lane)), __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (s0 + u < S) {
-          a0 += __uint_as_float(static_cast<uint32_t>(v[u]));
-          a1 += __uint_as_float(static_cast<uint32_t>(v[u] >> 32));
-        }
-    }
-    fwht128_wave(a0, a1);
-    const int64_t n0 = 128 * static_cast<int64_t>(g) + 2 * lane;
-    const float y0 = a0 * kRScale * static_cast<float>(svh[n0]);
-    const float y1 = a1 * kRScale * static_cast<float>(svh[n0 + 1]);
-    if (ydt == VYBDQ_F32) { store_elem<VYBDQ_F32>(Y, nullptr, b * N + n0, y0); store_elem<VYBDQ_F32>(Y, nullptr, b * N + n0 + 1, y1); }
-    else if (ydt == VYBDQ_F16) { store_elem<VYBDQ_F16>(Y, nullptr, b * N + n0, y0); store_elem<VYBDQ_F16>(Y, nullptr, b * N + n0 + 1, y1); }
-    else { store_elem<VYBDQ_BF16>(Y, nullptr, b * N + n0, y0); store_elem<VYBDQ_BF16>(Y, nullptr, b * N + n0 + 1, y1); }
+    for (int u = 0; u < 8; ++u)
+      if (s0 + u < S) {
+        a0 += __uint_as_float(static_cast<uint32_t>(v[u]));
+        a1 += __uint_as_float(static_cast<uint32_t>(v[u] >> 32));
+      }
   }
+  fwht128_wave(a0, a1);
+  const int64_t n0 = 128 * static_cast<int64_t>(g) + 2 * lane;
+  const float y0 = a0 * kRScale * static_cast<float>(svh[n0]);
+  const float y1 = a1 * kRScale * static_cast<float>(svh[n0 + 1]);
+  if (ydt == VYBDQ_F32) { store_elem<VYBDQ_F32>(Y, nullptr, b * N + n0, y0); store_elem<VYBDQ_F32>(Y, nullptr, b * N + n0 + 1, y1); }
+  else if (ydt == VYBDQ_F16) { store_elem<VYBDQ_F16>(Y, nullptr, b * N + n0, y0); store_elem<VYBDQ_F16>(Y, nullptr, b * N + n0 + 1, y1); }
+  else { store_elem<VYBDQ_BF16>(Y, nullptr, b * N + n0, y0); store_elem<VYBDQ_BF16>(Y, nullptr, b * N + n0 + 1, y1); }
 }
 
 // 3. (batch > 2) y[b][n] = svh[n] * FWHT(sum_s zpart[s][b][.]) / sqrt(128)
@@ -484,8 +315,14 @@ __global__ void __launch_bounds__(64) k_exl3_out(const float *__restrict__ zpart
 
 static int exl3_bp(int64_t B) { return B <= 1 ? 1 : B <= 2 ? 2 : B <= 4 ? 4 : B <= 8 ? 8 : 16; }
 
-// K-splits: enough workgroups to fill the chip, bounded so partials stay small; a split's
-// k-range is whole 128 chunks (the x rotation is done per chunk inside the GEMM)
+// K-splits: whole 128 chunks (the x rotation is done per chunk), and from 256 k on a multiple of 256
+// k, one 64-k step for each of the four waves. The product is bound by the decode on the VALU, so the
+// time follows the k-blocks that the fullest CU decodes: ceil(workgroups / CUs) * kbs, plus a little per
+// workgroup, per k-block of x rotated before the first step (batch <= 2) and per split of partials written
+// and read back (larger batches). Measured, batch 16: K = 5120, N = 17408: 5 splits (3 workgroups of
+// 64 k-blocks a CU) 25.8 us per call, 4 (3 x 80) 27.5, 7 (4 x 48) 26.2, 10 (6 x 32) 27.3; K = 17408, N = 5120:
+// 12 (2 x 96) 26.6, 17 (3 x 64) 28.1, 10 (2 x 112) 28.2, 14 (3 x 80) 29.6; K = 9216, N = 3072: 9 (1 x 64)
+// 17.6, 12 (2 x 48) 20.0. Batch 1, K = 17408: 12 splits 22.6, 10 24.4, 7 27.3 us.
 struct Exl3Split {
   int S;    // splits
   int kbs;  // 16-row k-blocks per split (a multiple of 8)
@@ -493,28 +330,33 @@ struct Exl3Split {
 static Exl3Split exl3_splits(int64_t K, int64_t N, int BP) {
   const int KB = static_cast<int>(K / 16);
   const int64_t groups = N / 128;
-  int S;
-  if (BP <= 2) {
-    // about 24 k-blocks per split (6 per wave), at most ~8 workgroups per CU. Measured, batch 1:
-    // K = 5120, N = 17408: 14 splits 20.2-20.9 us against 21.3-22.4 at 7-12; K = 10240: 14
-    // splits 37.4 us against 41.0 at 7; K = 2560: 7 splits 13.0 us against 13.7 at 10; K = 17408,
-    // N = 5120: 16 splits 24.8 us (12: 23.6, 7: 29.2). Fewer splits leave some CUs a workgroup
-    // more than others for longer; more add x rotations and partials.
-    S = (KB + 23) / 24;
-    const int64_t fill = groups < 2048 ? 2048 / groups : 1;
-    if (S > fill) S = static_cast<int>(fill);
-  } else {
-    // the matrix-core batches (4..16): ~2048 workgroups (K = 5120, N = 17408: batch 4 at 16 splits
-    // 1294 against 1194 GB/s at 8; batch 16: 8, 12, 20 and 24 splits 9-11% slower)
-    S = static_cast<int>((2048 + groups - 1) / groups);
+  auto shape = [&](int S) {
+    int kbs = (KB + S - 1) / S;
+    kbs = kbs > 8 ? (kbs + 15) / 16 * 16 : 8;
+    return Exl3Split{(KB + kbs - 1) / kbs, kbs};
+  };
+  Exl3Split best = shape(1);
+  int64_t best_cost = -1;
+  for (int S = 1; S <= 16; ++S) {
+    const Exl3Split c = shape(S);
+    const int64_t rounds = (groups * c.S + 255) / 256;
+    const int64_t cost = exl3_fused(BP) ? rounds * (8 * c.kbs + 16) + BP * c.kbs : rounds * (8 * c.kbs + 48) + 8 * c.S;
+    if (best_cost < 0 || cost < best_cost) best_cost = cost, best = c;
   }
-  if (S > 16) S = 16;
-  if (S > KB / 4) S = KB / 4 > 0 ? KB / 4 : 1;
-  if (const char *e = tuning_env("VYBDQ_EXL3_SPLITS")) S = atoi(e);  // tuning override
-  if (S < 1) S = 1;
-  int kbs = (KB + S - 1) / S;
-  kbs = (kbs + 7) / 8 * 8;
-  return {(KB + kbs - 1) / kbs, kbs};
+  if (const char *e = tuning_env("VYBDQ_EXL3_SPLITS")) best = shape(atoi(e) > 0 ? atoi(e) : 1);  // tuning override
+  return best;
+}
+
+// The sizes the entry takes: x' rows of one of at most 16 k-splits (a grid of 2048 workgroups) within
+// 160 KB, beside 40 KB of tiles above batch 2. (The kernel itself needs less.)
+static bool exl3_size_ok(int64_t K, int64_t N, int BP) {
+  const int64_t KB = K / 16, groups = N / 128;
+  int64_t S = exl3_fused(BP) ? (KB + 23) / 24 : (2048 + groups - 1) / groups;
+  if (exl3_fused(BP) && S > (groups < 2048 ? 2048 / groups : 1)) S = groups < 2048 ? 2048 / groups : 1;
+  S = S > 16 ? 16 : S;
+  S = S > KB / 4 ? KB / 4 : S;
+  const int64_t kbs = ((KB + S - 1) / S + 7) / 8 * 8;
+  return exl3_fused(BP) ? BP * 16 * kbs * 4 <= 160 * 1024 : BP * (16 * kbs + 8) * 2 + 40960 <= 160 * 1024;
 }
 
 // workspace: per-column-block arrival counters (zero between calls), x' (batch > 2), partials
@@ -593,18 +435,18 @@ extern "C" int64_t vybdq_exl3_workspace_size(int64_t B, int64_t K, int64_t N) {
   return exl3_ws_bytes(B, K, N);
 }
 
-template <int BP>
+template <bool FUSED>
 static void exl3_gemm_launch(const uint16_t *t, const void *X, int xdt, const _Float16 *su, const _Float16 *sv,
-                             void *Y, int ydt, int B, const _Float16 *xp, float *zp, uint32_t *arr, int64_t K,
+                             void *Y, int ydt, int B, int BP, const _Float16 *xp, float *zp, uint32_t *arr, int64_t K,
                              int NB, const Exl3Split &sp, hipStream_t s) {
-  const size_t lds = exl3_lds_bytes(BP, sp.kbs);  // <= 160 KB, checked by the caller
+  const size_t lds = exl3_lds_bytes(BP, sp.kbs);  // at most 82 KB (exl3_size_ok)
   if (lds > 64 * 1024) {
     static std::atomic<uint64_t> raised{0};
-    if (ensure_lds_limit(reinterpret_cast<const void *>(&k_exl3_gemm<BP>), 160 * 1024, raised, "exl3 gemm"))
+    if (ensure_lds_limit(reinterpret_cast<const void *>(&k_exl3_gemm<FUSED>), 160 * 1024, raised, "exl3 gemm"))
       return;  // the launch below then fails and check_launch reports it
   }
-  hipLaunchKernelGGL((k_exl3_gemm<BP>), dim3(static_cast<unsigned>(NB / 8), static_cast<unsigned>(sp.S)),
-                     dim3(256), lds, s, t, X, xdt, su, sv, Y, ydt, B, xp, zp, arr, K, NB, sp.kbs);
+  hipLaunchKernelGGL((k_exl3_gemm<FUSED>), dim3(static_cast<unsigned>(NB / 8), static_cast<unsigned>(sp.S)),
+                     dim3(256), lds, s, t, X, xdt, su, sv, Y, ydt, B, BP, xp, zp, arr, K, NB, sp.kbs);
 }
 
 extern "C" int vybdq_exl3_gemm(uint64_t trellis, uint64_t suh, uint64_t svh, uint64_t X, uint64_t Y, int64_t B,
@@ -622,7 +464,7 @@ extern "C" int vybdq_exl3_gemm(uint64_t trellis, uint64_t suh, uint64_t svh, uin
                 "workspace smaller than vybdq_exl3_workspace_size");
   const int BP = exl3_bp(B);
   const Exl3Split sp = exl3_splits(K, N, BP);
-  VYBDQ_REQUIRE(exl3_lds_bytes(BP, sp.kbs) <= 160 * 1024, VYBDQ_ERR_SHAPE,
+  VYBDQ_REQUIRE(exl3_size_ok(K, N, BP), VYBDQ_ERR_SHAPE,
                 "K too large for one split's x' stage in LDS at this batch");
   const int NB = static_cast<int>(N / 16);
   hipStream_t s = as_stream(stream);
@@ -636,16 +478,11 @@ extern "C" int vybdq_exl3_gemm(uint64_t trellis, uint64_t suh, uint64_t svh, uin
   void *y = reinterpret_cast<void *>(Y);
   const int b = static_cast<int>(B);
   if (!exl3_fused(BP)) {
-    const dim3 gx(static_cast<unsigned>(K / 128), static_cast<unsigned>(BP));
-    VYBDQ_DISPATCH_IN(x_dt, XDT, hipLaunchKernelGGL((k_exl3_xprep<XDT>), gx, dim3(64), 0, s, x, su, xp, b, K));
+    const dim3 gx(static_cast<unsigned>(K / 128), static_cast<unsigned>(B));
+    VYBDQ_DISPATCH_IN(x_dt, XDT, hipLaunchKernelGGL((k_exl3_xprep<XDT>), gx, dim3(64), 0, s, x, su, xp, K));
   }
-  switch (BP) {
-    case 1: exl3_gemm_launch<1>(t, x, x_dt, su, sv, y, y_dt, b, xp, zp, arr, K, NB, sp, s); break;
-    case 2: exl3_gemm_launch<2>(t, x, x_dt, su, sv, y, y_dt, b, xp, zp, arr, K, NB, sp, s); break;
-    case 4: exl3_gemm_launch<4>(t, x, x_dt, su, sv, y, y_dt, b, xp, zp, arr, K, NB, sp, s); break;
-    case 8: exl3_gemm_launch<8>(t, x, x_dt, su, sv, y, y_dt, b, xp, zp, arr, K, NB, sp, s); break;
-    default: exl3_gemm_launch<16>(t, x, x_dt, su, sv, y, y_dt, b, xp, zp, arr, K, NB, sp, s); break;
-  }
+  if (exl3_fused(BP)) exl3_gemm_launch<true>(t, x, x_dt, su, sv, y, y_dt, b, BP, xp, zp, arr, K, NB, sp, s);
+  else exl3_gemm_launch<false>(t, x, x_dt, su, sv, y, y_dt, b, BP, xp, zp, arr, K, NB, sp, s);
   if (!exl3_fused(BP)) {
     const dim3 go(static_cast<unsigned>(N / 128), static_cast<unsigned>(B));
     VYBDQ_DISPATCH_IN(y_dt, YDT, hipLaunchKernelGGL((k_exl3_out<YDT>), go, dim3(64), 0, s, zp, sv, y, BP, sp.S, N));

@@ -110,10 +110,126 @@ __device__ __forceinline__ void chunk_window(const u4 c, uint32_t (&w)[6]) {
   w[5] = c[3];
 }
 
-// One wave's LDS tile of decoded values for the matrix-core products: [128 columns][32 k] fp16,
-// column stride kExl3WtStride bytes (five 16-B slots: 16 consecutive columns fall on distinct banks)
-constexpr int kExl3WtStride = 80;
-constexpr int kExl3WtBytes = 128 * kExl3WtStride;  // one wave's tile
+// ---- trellis straight into matrix-core operands -------------------------------------------------
+//
+// A tile's stream dword 4 j + i (i = 0..3 of lane chunk j, its predecessor above it) holds the
+// windows of rows 2 i, 2 i + 1, 2 i + 8, 2 i + 9 of column j (shifts 28, 24, 20, 16) and of column
+// j + 8 (shifts 12, 8, 4, 0): the four words of either column, two fp16 halves each, are a lane's
+// whole B operand of v_mfma_f32_16x16x32_f16 (k' = 8 group + 2 row + half). So nothing is
+// regrouped through LDS and nothing is added or packed on the VALU: the matrix core adds x lo + x hi in
+// float32. Shifts s and s + 16 are the two halves of one funnel shift, so eight windows take three
+// of them. VALU instructions per weight: 2 hash products, 1 mask and xor, 3/8 windows = 3.4.
+
+// the eight windows of dword d (predecessor p), hashed up to their fp16 halves: a = column j, b = column j + 8
+__device__ __forceinline__ void dword_halves(uint32_t p, uint32_t d, u4 &a, u4 &b) {
+  auto fin = [](uint32_t x) { return (x & 0x8FFF8FFFu) ^ 0x3B603B60u; };
+  const uint32_t w12 = __builtin_amdgcn_alignbit(p, d, 12), w8 = __builtin_amdgcn_alignbit(p, d, 8),
+                 w4 = __builtin_amdgcn_alignbit(p, d, 4);
+  a = u4{fin(mcg_hash<true>(w12)), fin(mcg_hash<true>(w8)), fin(mcg_hash<true>(w4)), fin(mcg_hash<true>(d))};
+  b = u4{fin(mcg_hash<false>(w12)), fin(mcg_hash<false>(w8)), fin(mcg_hash<false>(w4)), fin(mcg_hash<false>(d))};
+}
+
+constexpr int kExl3Step = 4;  // k-blocks of 16 rows per step of exl3_mma_run
+
+// A workgroup barrier for LDS alone: waits for this wave's LDS accesses, not for its loads in flight
+// (the release fence of __syncthreads() may wait for those).
+__device__ __forceinline__ void exl3_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+}
+
+// One wave: acc += x' (at most 16 rows) times `nsteps` steps of 64 k of 128 columns (eight tiles per
+// k-block). Lane l: k-block l >> 4 of the step, chunk l & 7 of the tile pair's tile (l >> 3) & 1, so
+// each 16-byte load instruction covers 256 contiguous bytes of four k-blocks, the four pairs of a
+// step whole 1 KB runs. `base`: the first step's first tile (wave-uniform); `kstride`: uint16 from
+// one k-block to the next; aload(st, v): step st's 16 x' values (k-block l >> 4 of the step) of row
+// l & 15 (any finite or other values for rows past the group: they reach only outputs that are not
+// stored), two steps ahead if AHEAD (x' in memory) or at the step (x' in LDS); ready() runs between the first trellis loads and the first aload (it may stage x' in LDS and
+// wait for it: the trellis loads stay in flight across an exl3_barrier). acc[2 c + h][r] = z[row 4 (l >> 4) + r][exl3_mma_col(c, h, l)]. Two steps of loads are in
+// flight per lane (8 KB per wave); each ring slot is refilled right after its use, pinned by
+// scheduling barriers (sunk to the end of the step it would leave no load in flight).
+template <bool AHEAD, class Ready, class ALoad>
+__device__ __forceinline__ void exl3_mma_run(const uint16_t *__restrict__ base, int64_t kstride, int nsteps,
+                                             const Ready &ready, const ALoad &aload, f4 (&acc)[8]) {
+  if (nsteps <= 0) {
+    ready();
+    return;
+  }
+  const int lane = threadIdx.x & 63, n = lane & 15;
+  const uint16_t *lp = base + (lane >> 4) * kstride + 8 * n;
+  constexpr int R = 2;
+  u4 ring[R][4], xr[AHEAD ? R : 1][2];
+  auto wload = [&](int st, int c) {
+    const int sc = st < nsteps ? st : nsteps - 1;  // in range: re-read the last
+    return *reinterpret_cast<const u4 *>(lp + kExl3Step * kstride * sc + 128 * c);
+  };
+#pragma unroll
+  for (int d = 0; d < R; ++d)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) ring[d][c] = wload(d, c);
+  __builtin_amdgcn_sched_barrier(0);
+  ready();
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int d = 0; d < R; ++d) aload(d < nsteps ? d : nsteps - 1, xr[d]);
+  }
+  auto step = [&](int st, u4 (&rw)[4], u4 (&rx)[2]) {
+    if constexpr (!AHEAD) aload(st, rx);
+    // A of dword i: rows 2 i, 2 i + 1, 2 i + 8, 2 i + 9 of the lane's k-block, each value twice
+    h8 a[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      a[i] = __builtin_bit_cast(h8, u4{__builtin_amdgcn_perm(rx[0][i], rx[0][i], 0x01000100u),
+                                       __builtin_amdgcn_perm(rx[0][i], rx[0][i], 0x03020302u),
+                                       __builtin_amdgcn_perm(rx[1][i], rx[1][i], 0x01000100u),
+                                       __builtin_amdgcn_perm(rx[1][i], rx[1][i], 0x03020302u)});
+    if constexpr (AHEAD) aload(st + R < nsteps ? st + R : nsteps - 1, rx);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      uint32_t w[6];
+      chunk_window(rw[c], w);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        u4 b0, b1;
+        dword_halves(w[i + 1], w[i + 2], b0, b1);
+        acc[2 * c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], __builtin_bit_cast(h8, b0), acc[2 * c], 0, 0, 0);
+        acc[2 * c + 1] =
+            __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], __builtin_bit_cast(h8, b1), acc[2 * c + 1], 0, 0, 0);
+      }
+      rw[c] = wload(st + R, c);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  int st = 0;
+  for (; st + R <= nsteps; st += R) {
+#pragma unroll
+    for (int d = 0; d < R; ++d) step(st + d, ring[d], xr[AHEAD ? d : 0]);
+  }
+  if (st < nsteps) step(st, ring[0], xr[0]);
+}
+
+// column (of the 128) of accumulator 2 c + h in lane l
+__device__ __forceinline__ int exl3_mma_col(int c, int h, int l) {
+  return 32 * c + 16 * ((l >> 3) & 1) + (l & 7) + 8 * h;
+}
+
+// the wave's accumulators to its rows of the workgroup's partials [4 waves][rows][kExl3RedStride];
+// rows past B are not written
+constexpr int kExl3RedStride = 132;  // 4 floats of padding: the four row groups fall on different banks
+__device__ __forceinline__ void exl3_mma_store(const f4 (&acc)[8], float *red, int B) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int b = 4 * (lane >> 4) + r;
+    if (b < B)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) red[b * kExl3RedStride + exl3_mma_col(q >> 1, q & 1, lane)] = acc[q][r];
+  }
+}
 
 // ---- 128-point FWHT across a wave (2 elements per lane) -------------------------------------
 

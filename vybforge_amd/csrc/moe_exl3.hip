@@ -10,15 +10,14 @@
 //
 // Here on the stream, with no host loop, no host synchronisation and no dequantized copy of any
 // weight (x W = svh * FWHT(FWHT(x * suh)/sqrt(128) What)/sqrt(128) per 128 chunk):
-//  1. route + bucket (moe.hip): rows = (token, slot) pairs grouped by expert; groups of <= BP rows.
+//  1. route + bucket (moe.hip): rows = (token, slot) pairs grouped by expert; groups of at most 16
+//     rows of one expert (of one row at one token).
 //  2. k_mx_xprep: x'[p][row] = FWHT(x[token] * suh_{e,p}) / sqrt(128), p = gate, up, stored as fp16
 //     after a power-of-two scale per row that brings its largest |x'| into [2^14, 2^15) (exact;
 //     multiplied back after the product, which is linear in x'): no overflow, no fp16 subnormals.
 //  3. k_mx_gemm: z[split][row][p I + n] = sum over the split's k of x'[p][row][k] What_{e,p}[k][n];
-//     the trellis is decoded in registers with the mcg hash exactly as in the fused GEMM
-//     (exl3_dev.h): row groups of one or two rows dot the two fp16 halves of each value with
-//     (x', x') pairs; larger groups write the decoded values to a per-wave LDS tile and multiply
-//     on the matrix cores, with the x' rows read straight from the workspace as the A operand.
+//     the trellis is hashed in registers straight into matrix-core operands (exl3_dev.h), with the
+//     x' rows read from the workspace as the A operand.
 //  4. k_mx_mid: g, u = FWHT(sum_split z)/sqrt(128) * svh; a = silu(min(g, L)) * clamp(u, -L, L);
 //     a' = FWHT(a * suh_down)/sqrt(128) per row, stored as fp16 with its own power-of-two row scale
 //     (a' is small: activations times suh, and subnormal in fp16 without it).
@@ -296,7 +295,7 @@ __global__ void __launch_bounds__(256) k_bf16_terms(const void *__restrict__ X, 
 struct MxGemmArgs {
   const uint64_t *tab;
   int proj0;           // table projection of the first output block: 0 (gate | up) or 2 (down)
-  const int4 *groups;  // {expert, r0, r1, 0}: rows [r0, r1) of one expert, at most BP
+  const int4 *groups;  // {expert, r0, r1, 0}: rows [r0, r1) of one expert, at most 16
   const int *ngroups;
   const _Float16 *xp;  // [nproj][rows][K] rotated inputs
   int rows;            // rows of the bucketing (T topk)
@@ -306,29 +305,23 @@ struct MxGemmArgs {
   int ncat;            // nproj Np
   int kbs;             // 16-row k-blocks per split (a multiple of 8)
   int gy;              // grid y of the routed column blocks; shared-expert workgroups follow
+  int red_rows;        // rows of the waves' partials in LDS (the largest group)
 };
 
-constexpr int kMxRedStride = 132;  // floats per row of the per-wave partials (16-column groups on distinct banks)
-
-__host__ __device__ constexpr size_t mx_lds_bytes(int BP, int kbs) {
-  // BP <= 2: the split's (x', x') pairs; larger: one decoded-value tile per wave; both reused for
-  // the per-wave partials [4][BP][kMxRedStride] after the loop
-  return (BP <= 2 ? static_cast<size_t>(BP) * 16 * kbs * 4 : static_cast<size_t>(4) * kExl3WtBytes) >
-                 static_cast<size_t>(4) * BP * kMxRedStride * 4
-             ? (BP <= 2 ? static_cast<size_t>(BP) * 16 * kbs * 4 : static_cast<size_t>(4) * kExl3WtBytes)
-             : static_cast<size_t>(4) * BP * kMxRedStride * 4;
-}
-
 // grid (groups bound rounded to 8, nproj Np / 128 column blocks, S splits), 4 waves: each wave a
-// quarter of the split's k-blocks on the block's 128 columns, the waves' partials summed in LDS in
-// a fixed order. The group index is the fastest grid dimension and the bound is a multiple of 8,
-// so every column block of one group runs on the same XCD (its L2 holds the group's x' rows).
+// quarter of the split's 64-k steps on the block's 128 columns (exl3_mma_run: the trellis goes from
+// registers straight into matrix-core operands), x' read from the workspace (L2), the waves'
+// partials summed in LDS in a fixed order. The group index is the fastest grid dimension and the
+// bound is a multiple of 8, so every column block of one group runs on the same XCD (its L2 holds
+// the group's x' rows). Bound by the hash on the VALU (4.0 instructions per weight, 82% of the issue
+// slots). 256 tokens, H = 4096, I = 2048, 288 experts: gate | up 735 us, down 426 us (995 and 563 with the
+// decoded words regrouped through LDS, 7.3 instructions per weight).
 // SH: the launch also carries the shared expert's tiles (0 none; 1 gate | up, bf16 activations;
-// 2 gate | up, activations as bf16 hi + lo terms; 3 down, hi + lo), as workgroups with blockIdx.x
-// past the routed groups' bound: its bf16 weights stream from HBM while the routed workgroups
+// 2 gate | up, activations as bf16 hi + lo terms; 3 down, hi + lo), as workgroups with blockIdx.y
+// past the routed column blocks: its bf16 weights stream from HBM while the routed workgroups
 // decode trellis on the VALU.
-template <int BP, int SH>
-__global__ void __launch_bounds__(256) k_mx_gemm(const MxGemmArgs a, const MxShared sh) {
+template <int SH>
+__global__ void __launch_bounds__(256, 4) k_mx_gemm(const MxGemmArgs a, const MxShared sh) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int jt = blockIdx.x;
   if constexpr (SH != 0) {
@@ -343,191 +336,41 @@ __global__ void __launch_bounds__(256) k_mx_gemm(const MxGemmArgs a, const MxSha
   }
   if (jt >= *a.ngroups) return;
   const int4 grp = a.groups[jt];
-  const int e = grp.x, r0 = grp.y, B = grp.z - grp.y;  // 1 <= B <= BP
+  const int e = grp.x, r0 = grp.y, B = grp.z - grp.y;  // 1 <= B <= 16
   const int nbp = a.Np / 128;
   const int p = static_cast<int>(blockIdx.y) / nbp, g = static_cast<int>(blockIdx.y) - p * nbp;
   const int s = blockIdx.z;
-  const uint16_t *__restrict__ trellis = mx_ptr<uint16_t>(a.tab, e, a.proj0 + p, 0);
-  const int NB = a.Np / 16;
-  const int64_t K = a.K;
-  const int KB = static_cast<int>(K / 16);
+  const int64_t K = a.K, kstride = static_cast<int64_t>(a.Np) * 4;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  const int t = lane >> 3, j = lane & 7;
   const int kb_begin = s * a.kbs;
-  const int kb_end = min(kb_begin + a.kbs, KB);
-  const int nkb = kb_end - kb_begin;  // a multiple of 8 (K % 128 == 0)
-  constexpr bool HALVES = BP <= 2;
-  constexpr int kD = 4;  // trellis chunks in flight per lane
-  const int per_wave = (nkb + 3) / 4;  // even: wave ranges start at even k-blocks
-  const int w_begin = wave * per_wave;
-  const int w_end = min(w_begin + per_wave, nkb);
-  const int64_t nb = 8 * static_cast<int64_t>(g) + t;
-  auto load_chunk = [&](int kk) {
-    const int kc = kk < w_end ? kk : (w_end > w_begin ? w_end - 1 : 0);  // in range: re-read the last
-    const int64_t tile = static_cast<int64_t>(kb_begin + kc) * NB + nb;
-    return *reinterpret_cast<const u4 *>(trellis + tile * 64 + 8 * j);
-  };
-  // this group's x' rows from the split's first k
-  const _Float16 *xsrc = a.xp + (static_cast<int64_t>(p) * a.rows + r0) * K + 16 * static_cast<int64_t>(kb_begin);
-  const int krows = 16 * nkb;
-
-  // BP <= 2: the rows' (x', x') pairs of the split in LDS; rows past the group read as zero. All
-  // of a thread's 16-byte reads (at most 8: the stage holds at most 64 KB, nc <= 2048) go out
-  // before the trellis ring (loads return in order), and none after it: x loads issued after the
-  // ring (a staging loop) made the compiler wait for the whole ring at the top of every k-loop
-  // iteration.
-  const int per_row = krows / 8;
-  const int nc = HALVES ? BP * per_row : 0;
-  auto x_chunk = [&](int i) {
-    const int b = i / per_row, c = i - b * per_row;
-    u4 v = u4{0u, 0u, 0u, 0u};
-    if (b < B) v = *reinterpret_cast<const u4 *>(xsrc + b * K + 8 * c);
-    return v;
-  };
-  auto x_store = [&](int i, const u4 v) {
-    const int b = i / per_row, c = i - b * per_row;
-    u4 *d = reinterpret_cast<u4 *>(reinterpret_cast<uint32_t *>(smem) + b * krows + 8 * c);
-    auto dup = [](uint32_t h) { return (h & 0xffffu) | (h << 16); };
-    d[0] = u4{dup(v[0]), dup(v[0] >> 16), dup(v[1]), dup(v[1] >> 16)};
-    d[1] = u4{dup(v[2]), dup(v[2] >> 16), dup(v[3]), dup(v[3] >> 16)};
-  };
-  constexpr int XV = HALVES ? 8 : 1;
-  u4 xv[XV];
-  if constexpr (HALVES) {
-#pragma unroll
-    for (int u = 0; u < XV; ++u) {
-      const int i = threadIdx.x + 256 * u;
-      if (i < nc) xv[u] = x_chunk(i);
-    }
-  }
-  // larger groups: the matrix-core A values of k-block kk: x' row lane & 15 (zero past the group),
-  // k offset 4 (lane >> 4), four fp16 read from the workspace (L2) one group of kD k-blocks ahead,
-  // beside the trellis ring (each is used twice in the A fragment, see step)
+  const int nst = (min(kb_begin + a.kbs, static_cast<int>(K / 16)) - kb_begin) / kExl3Step;  // K % 128 == 0
+  const int st0 = nst * wave / 4, st1 = nst * (wave + 1) / 4;
+  const int kb0 = kb_begin + kExl3Step * st0;
   const int am = lane & 15;
-  const _Float16 *arow = xsrc + static_cast<int64_t>(am < B ? am : 0) * K + 4 * (lane >> 4);
-  auto load_a = [&](int kk) {
-    u2 v = u2{0u, 0u};
-    const int kc = kk < w_end ? kk : w_begin;
-    if (am < B) v = *reinterpret_cast<const u2 *>(arow + 16 * kc);
-    return v;
-  };
-  __builtin_amdgcn_sched_barrier(0);
-  u4 ring[kD];
-  u2 aring[HALVES ? 1 : kD];
-  if constexpr (HALVES) aring[0] = u2{0u, 0u};
+  const _Float16 *arow = a.xp + (static_cast<int64_t>(p) * a.rows + r0 + (am < B ? am : 0)) * K +
+                         16 * static_cast<int64_t>(kb0 + (lane >> 4));
+  f4 acc[8];
 #pragma unroll
-  for (int d = 0; d < kD; ++d) {
-    ring[d] = load_chunk(w_begin + d);
-    if constexpr (!HALVES) aring[d] = load_a(w_begin + d);
-  }
-  if constexpr (HALVES) {
-#pragma unroll
-    for (int u = 0; u < XV; ++u)
-      if (threadIdx.x + 256 * u < nc) x_store(threadIdx.x + 256 * u, xv[u]);
-    __syncthreads();
-  }
-
-  float acc[BP][2];
-#pragma unroll
-  for (int b = 0; b < BP; ++b) acc[b][0] = acc[b][1] = 0.f;
-  f4 accm[HALVES ? 1 : 8];
-#pragma unroll
-  for (int f = 0; f < (HALVES ? 1 : 8); ++f) accm[f] = f4{0.f, 0.f, 0.f, 0.f};
-  char *wt = smem + static_cast<size_t>(wave) * kExl3WtBytes;
-  auto step = [&](int kk, const u4 c, const u2 av) {
-    uint32_t w[6];
-    chunk_window(c, w);
-    if constexpr (HALVES) {
-      uint32_t xq[BP][16];
-#pragma unroll
-      for (int b = 0; b < BP; ++b) {
-        const u4 *src = reinterpret_cast<const u4 *>(reinterpret_cast<const uint32_t *>(smem) + b * krows + 16 * kk);
-#pragma unroll
-        for (int c4 = 0; c4 < 4; ++c4) {
-          const u4 v4 = src[c4];
-          xq[b][4 * c4 + 0] = v4[0];
-          xq[b][4 * c4 + 1] = v4[1];
-          xq[b][4 * c4 + 2] = v4[2];
-          xq[b][4 * c4 + 3] = v4[3];
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < 32; ++q) {
-        const h2 y = __builtin_bit_cast(h2, slot_halves(w, q));
-#pragma unroll
-        for (int b = 0; b < BP; ++b)
-          acc[b][q >> 4] = __builtin_amdgcn_fdot2(y, __builtin_bit_cast(h2, xq[b][q & 15]), acc[b][q >> 4], false);
-      }
-    } else {
-      // the 32 slot words as they are (two fp16 halves per value, whose sum is the value): column
-      // c's 16 words in k order are the tile row [c][k' = 2 k + h], and the MFMA with each x'
-      // value twice in A adds x lo + x hi in float32 (as the k_exl3_gemm matrix-core path)
-      const int c0 = 16 * t + j;
-      uint32_t hw[32];
-#pragma unroll
-      for (int q = 0; q < 32; ++q) hw[q] = slot_halves(w, q);
-      u4 *d0 = reinterpret_cast<u4 *>(wt + c0 * kExl3WtStride);
-      u4 *d1 = reinterpret_cast<u4 *>(wt + (c0 + 8) * kExl3WtStride);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        d0[i] = u4{hw[4 * i], hw[4 * i + 1], hw[4 * i + 2], hw[4 * i + 3]};
-        d1[i] = u4{hw[16 + 4 * i], hw[16 + 4 * i + 1], hw[16 + 4 * i + 2], hw[16 + 4 * i + 3]};
-      }
-      const h8 a = __builtin_bit_cast(h8, u4{__builtin_amdgcn_perm(av[0], av[0], 0x01000100u),
-                                             __builtin_amdgcn_perm(av[0], av[0], 0x03020302u),
-                                             __builtin_amdgcn_perm(av[1], av[1], 0x01000100u),
-                                             __builtin_amdgcn_perm(av[1], av[1], 0x03020302u)});
-      const int gk = lane >> 4;
-#pragma unroll
-      for (int f = 0; f < 8; ++f) {
-        const h8 bw = *reinterpret_cast<const h8 *>(wt + (16 * f + am) * kExl3WtStride + 16 * gk);
-        accm[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bw, accm[f], 0, 0, 0);
-      }
-    }
-  };
-  // Whole groups of kD k-blocks, each ring slot (trellis chunk and A values) refilled right after the
-  // step that consumed it; the last blocks are in the ring.
-  int k0 = w_begin;
-  for (; k0 + kD <= w_end; k0 += kD) {
-#pragma unroll
-    for (int d = 0; d < kD; ++d) {
-      step(k0 + d, ring[d], aring[HALVES ? 0 : d]);
-      ring[d] = load_chunk(k0 + d + kD);
-      if constexpr (!HALVES) aring[d] = load_a(k0 + d + kD);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-#pragma unroll
-  for (int d = 0; d < kD - 1; ++d)
-    if (k0 + d < w_end) step(k0 + d, ring[d], aring[HALVES ? 0 : d]);
+  for (int f = 0; f < 8; ++f) acc[f] = f4{0.f, 0.f, 0.f, 0.f};
+  exl3_mma_run<true>(mx_ptr<uint16_t>(a.tab, e, a.proj0 + p, 0) + kb0 * kstride + 512 * g, kstride, st1 - st0,
+               [] {},
+               [&](int st, u4 (&v)[2]) {
+                 const u4 *x = reinterpret_cast<const u4 *>(arow + 16 * kExl3Step * st);
+                 v[0] = x[0];
+                 v[1] = x[1];
+               },
+               acc);
 
   // reduce the 4 waves (same columns, different k) in a fixed order, then this split's partial
-  __syncthreads();
-  float *red = reinterpret_cast<float *>(smem);  // [4][BP][kMxRedStride]
-  if constexpr (!HALVES) {
-    // accm[f][r] = z[row 4 (lane >> 4) + r][column 16 f + (lane & 15)]
-#pragma unroll
-    for (int f = 0; f < 8; ++f)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int b = 4 * (lane >> 4) + r;
-        if (b < BP) red[(wave * BP + b) * kMxRedStride + 16 * f + (lane & 15)] = accm[f][r];
-      }
-  } else {
-    const int c0 = 16 * t + j;  // this lane's columns: c0 and c0 + 8
-#pragma unroll
-    for (int b = 0; b < BP; ++b) {
-      red[(wave * BP + b) * kMxRedStride + c0] = acc[b][0];
-      red[(wave * BP + b) * kMxRedStride + c0 + 8] = acc[b][1];
-    }
-  }
+  float *red = reinterpret_cast<float *>(smem);  // [4][rows][kExl3RedStride]
+  const int wst = a.red_rows * kExl3RedStride;
+  exl3_mma_store(acc, red + wave * wst, B);
   __syncthreads();
   float *zo = a.zpart + (static_cast<int64_t>(s) * a.rows + r0) * a.ncat + static_cast<int64_t>(p) * a.Np + 128 * g;
   for (int i = threadIdx.x; i < B * 128; i += 256) {
     const int b = i >> 7, c = i & 127;
-    zo[static_cast<int64_t>(b) * a.ncat + c] =
-        ((red[(0 * BP + b) * kMxRedStride + c] + red[(1 * BP + b) * kMxRedStride + c]) +
-         red[(2 * BP + b) * kMxRedStride + c]) + red[(3 * BP + b) * kMxRedStride + c];
+    const float *o = red + b * kExl3RedStride + c;
+    zo[static_cast<int64_t>(b) * a.ncat + c] = ((o[0] + o[wst]) + o[2 * wst]) + o[3 * wst];
   }
 }
 
@@ -689,19 +532,16 @@ __global__ void __launch_bounds__(64 * kMxRowWaves) k_mx_combine(const uint64_t 
 
 // ---- host ---------------------------------------------------------------------------------------
 
-// rows per group: one per expert at one token (every expert then holds one row), two while the
-// experts hit average at most two rows, else 16-row groups on the matrix cores
-static int mx_bp(int64_t T, int64_t E, int64_t k) {
-  const int64_t n = T * k, hit = E < n ? E : n;
-  if (T == 1) return 1;
-  return n <= 2 * hit ? 2 : 16;
-}
+// rows per group: one at one token (every expert then holds one row), else 16 (the rows of one MFMA:
+// a group of more rows decodes its expert once for all of them)
+static int mx_bp(int64_t T) { return T == 1 ? 1 : 16; }
 
-// K splits of a grouped product: ~2048 workgroups over the expected groups, whole 128 chunks
+// K splits of a grouped product: ~2048 workgroups over the expected groups (one token: 512 to 3072 within
+// 2%, two tokens 84 to 91 us, four 139 to 144)
 struct MxSplit {
   int S, kbs;
 };
-static MxSplit mx_splits(int64_t K, int64_t groups, int64_t col_blocks, int BP) {
+static MxSplit mx_splits(int64_t K, int64_t groups, int64_t col_blocks) {
   const int KB = static_cast<int>(K / 16);
   const int64_t units = groups * col_blocks;
   int64_t target = 2048;  // workgroups (VYBDQ_MX_WGS overrides)
@@ -711,9 +551,7 @@ static MxSplit mx_splits(int64_t K, int64_t groups, int64_t col_blocks, int BP) 
   if (S > KB / 8) S = KB / 8;
   if (S < 1) S = 1;
   int kbs = (KB + S - 1) / S;
-  kbs = (kbs + 7) / 8 * 8;
-  // the (x', x') stage of a split in LDS (BP <= 2): at most 64 KB
-  while (BP <= 2 && mx_lds_bytes(BP, kbs) > 64 * 1024) kbs -= 8;
+  kbs = kbs > 8 ? (kbs + 15) / 16 * 16 : 8;  // whole 64-k steps for each of the four waves
   return {(KB + kbs - 1) / kbs, kbs};
 }
 
@@ -737,12 +575,12 @@ struct MxPlan {
 
 static MxPlan mx_plan(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k) {
   MxPlan p{};
-  p.BP = mx_bp(T, E, k);
+  p.BP = mx_bp(T);
   const int64_t n = T * k, hit = E < n ? E : n;
-  const int64_t groups = p.BP == 16 ? hit + n / 16 : (p.BP == 2 ? (n + 1) / 2 : n);
+  const int64_t groups = p.BP == 1 ? n : hit + n / 16;
   p.max_groups = static_cast<int>((moe_tiles_bound(T, E, k, p.BP) + 7) / 8 * 8);
-  p.gu = mx_splits(H, groups, 2 * I / 128, p.BP);
-  p.dn = mx_splits(I, groups, H / 128, p.BP);
+  p.gu = mx_splits(H, groups, 2 * I / 128);
+  p.dn = mx_splits(I, groups, H / 128);
   p.Ssg = bf16_splits(H, I, T, p.kps_g);
   p.Ssd = bf16_splits(I, H, T, p.kps_d);
   return p;
@@ -793,34 +631,25 @@ static MxWs mx_layout(char *base, const MxPlan &p, int64_t T, int64_t H, int64_t
   return m;
 }
 
-template <int BP, int SH>
+template <int SH>
 static int mx_gemm_launch(const MxGemmArgs &a, const MxShared &sh, int nproj, int S, int max_groups, hipStream_t s) {
-  const size_t lds = mx_lds_bytes(BP, a.kbs);
+  const size_t lds = static_cast<size_t>(4) * a.red_rows * kExl3RedStride * 4;  // 33 KB at 16 rows
   const unsigned gx = static_cast<unsigned>(max_groups), gz = static_cast<unsigned>(S);
   const unsigned extra = SH ? static_cast<unsigned>((sh.tiles + gx * gz - 1) / (gx * gz)) : 0u;
   MxGemmArgs b = a;
   b.gy = nproj * a.Np / 128;
-  hipLaunchKernelGGL((k_mx_gemm<BP, SH>), dim3(gx, static_cast<unsigned>(b.gy) + extra, gz), dim3(256), lds, s, b, sh);
+  hipLaunchKernelGGL((k_mx_gemm<SH>), dim3(gx, static_cast<unsigned>(b.gy) + extra, gz), dim3(256), lds, s, b, sh);
   return check_launch("moe exl3 grouped product");
 }
 
 // the grouped product of the routed experts, carrying the shared expert's tiles of kind SH
-template <int BP>
-static int mx_gemm_bp(int SH, const MxGemmArgs &a, const MxShared &sh, int nproj, int S, int max_groups,
-                      hipStream_t s) {
+static int mx_gemm(int SH, const MxGemmArgs &a, const MxShared &sh, int nproj, int S, int max_groups, hipStream_t s) {
   switch (SH) {
-    case 1: return mx_gemm_launch<BP, 1>(a, sh, nproj, S, max_groups, s);
-    case 2: return mx_gemm_launch<BP, 2>(a, sh, nproj, S, max_groups, s);
-    case 3: return mx_gemm_launch<BP, 3>(a, sh, nproj, S, max_groups, s);
-    default: return mx_gemm_launch<BP, 0>(a, sh, nproj, S, max_groups, s);
+    case 1: return mx_gemm_launch<1>(a, sh, nproj, S, max_groups, s);
+    case 2: return mx_gemm_launch<2>(a, sh, nproj, S, max_groups, s);
+    case 3: return mx_gemm_launch<3>(a, sh, nproj, S, max_groups, s);
+    default: return mx_gemm_launch<0>(a, sh, nproj, S, max_groups, s);
   }
-}
-
-static int mx_gemm(int BP, int SH, const MxGemmArgs &a, const MxShared &sh, int nproj, int S, int max_groups,
-                   hipStream_t s) {
-  if (BP == 1) return mx_gemm_bp<1>(SH, a, sh, nproj, S, max_groups, s);
-  if (BP == 2) return mx_gemm_bp<2>(SH, a, sh, nproj, S, max_groups, s);
-  return mx_gemm_bp<16>(SH, a, sh, nproj, S, max_groups, s);
 }
 
 }  // namespace vybdq
@@ -895,6 +724,7 @@ extern "C" int vybdq_moe_forward_exl3(uint64_t x, int x_dt, uint64_t logits, int
   ga.Np = static_cast<int>(I);
   ga.ncat = static_cast<int>(2 * I);
   ga.kbs = p.gu.kbs;
+  ga.red_rows = p.BP;
   // the shared expert's gate | up ride on this launch, its SwiGLU on the mid launch, its down
   // projection on the down launch (bf16 weights on the matrix cores: activations that are not
   // bf16 enter as two bf16 terms hi + lo, 16 significant bits)
@@ -938,7 +768,7 @@ extern "C" int vybdq_moe_forward_exl3(uint64_t x, int x_dt, uint64_t logits, int
     shd.S = p.Ssd;
     shd.tiles = shd.ngx * p.Ssd * static_cast<int>((T + 15) / 16);
   }
-  rc = mx_gemm(p.BP, shared ? (lo ? 2 : 1) : 0, ga, shg, 2, p.gu.S, p.max_groups, s);
+  rc = mx_gemm(shared ? (lo ? 2 : 1) : 0, ga, shg, 2, p.gu.S, p.max_groups, s);
   if (rc) return rc;
   // 4. SwiGLU between the rotations
   MxSwiglu sw{m.sgu, p.Ssg, static_cast<int>(T), static_cast<int>(I), m.ah, m.al};
@@ -959,7 +789,7 @@ extern "C" int vybdq_moe_forward_exl3(uint64_t x, int x_dt, uint64_t logits, int
   da.Np = static_cast<int>(H);
   da.ncat = static_cast<int>(H);
   da.kbs = p.dn.kbs;
-  rc = mx_gemm(p.BP, shared ? 3 : 0, da, shd, 1, p.dn.S, p.max_groups, s);
+  rc = mx_gemm(shared ? 3 : 0, da, shd, 1, p.dn.S, p.max_groups, s);
   if (rc) return rc;
   // 7. combine
   // four chunks per workgroup once the grid holds 2048 workgroups with them, else one
