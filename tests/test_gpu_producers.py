@@ -29,6 +29,25 @@ def test_rmsnorm_q8(dev, xdt, M, N):
     np.testing.assert_array_equal(Xs.cpu().numpy(), d)
 
 
+@pytest.mark.parametrize("M,N", [(1, 288), (5, 2592), (200, 544), (511, 256), (600, 1056)])
+def test_rmsnorm_q8_row_parts(dev, M, N):
+    """Rows split over workgroups (ragged last part, several 256-column chunks per part, unsplit) and the same rows
+    written over their input (Y and X one buffer: the unsplit kernel): bit-equal to the oracle."""
+    rng = np.random.default_rng(M + N)
+    x = torch.from_numpy(rng.standard_normal((M, N)).astype(np.float32))
+    w = torch.from_numpy(rng.uniform(0.5, 1.5, N).astype(np.float32))
+    _, y32, q, d = producers.rms_norm(x.double().numpy(), w.double().numpy(), 1e-6)
+    xd, wd = x.to(dev), w.to(dev)
+    _, Y32, Xq, Xs = ops.rmsnorm_q8(xd, wd, 1e-6, f32_copy=True)
+    rc = _lib.lib.vybdq_rmsnorm_q8(xd.data_ptr(), wd.data_ptr(), xd.data_ptr(), 0, 0, 0, M, N, 1e-6, 0, 0,
+                                   torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    for got in (Y32, xd):
+        np.testing.assert_array_equal(got.cpu().numpy(), y32)
+    np.testing.assert_array_equal(Xq.cpu().numpy(), q)
+    np.testing.assert_array_equal(Xs.cpu().numpy(), d)
+
+
 def test_rmsnorm_outputs_optional_and_16bit(dev):
     """Only a 16-bit Y (no float32 copy, no q8), N not a multiple of 32; large and tiny rows
     (the Newton seed range ends at 1e-9 and 1e9)."""

@@ -16,6 +16,8 @@
 //    32-lane half of a wave) a = max|x|, d = a / 127, q = sat_s8(rint(x * 127 / a)).
 #include "common.h"
 
+#include <utility>
+
 namespace vybdq {
 
 template <int DT>
@@ -174,6 +176,61 @@ __global__ void __launch_bounds__(256) k_rms_q8(const void *__restrict__ X, cons
   }
 }
 
+// The same row split over `parts` workgroups: each sums the whole row (the same threads, order and
+// fold, so the same r bit for bit) and writes its own E elements (a multiple of 256), one per thread at
+// a time: a short loop, because the unrolled row of the kernel above is ~20 KB of code that a decode
+// graph fetches anew on every launch (one row of 5120 in such a graph: 22.4 us, here 5).
+template <int XDT>
+__global__ void __launch_bounds__(256) k_rms_q8_parts(const void *__restrict__ X, const void *__restrict__ W,
+                                                      void *__restrict__ Y, int ydt, float *__restrict__ Y32,
+                                                      int8_t *__restrict__ Xq, float *__restrict__ Xs, int64_t N,
+                                                      int64_t E, double eps) {
+#pragma clang fp contract(off)
+  __shared__ double part[256];
+  __shared__ double rsh;
+  const int t = threadIdx.x;
+  const int64_t base = static_cast<int64_t>(blockIdx.y) * N;
+  const int64_t e0 = static_cast<int64_t>(blockIdx.x) * E, e1 = e0 + E < N ? e0 + E : N;
+  // the first elements to write, loaded with the sum's
+  const int64_t f = e0 + t < N ? e0 + t : N - 1;
+  double xf = load_d<XDT>(X, base + f), wf = load_d<XDT>(W, f);
+  constexpr int U = 8;
+  double ss = 0.0;
+  for (int64_t d0 = t; d0 < N; d0 += 256 * U) {
+    double v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = load_d<XDT>(X, base + (d0 + 256 * u < N ? d0 + 256 * u : N - 1));
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (d0 + 256 * u < N) ss = ss + v[u] * v[u];
+  }
+  part[t] = ss;
+  __syncthreads();
+  if (t < 128) part[t] = part[t] + part[t + 128];
+  __syncthreads();
+  if (t < 64) {
+    double sw = part[t] + part[t + 64];
+#pragma unroll
+    for (int st = 32; st > 0; st >>= 1) sw = sw + __shfl_down(sw, st, 64);
+    if (t == 0) rsh = 1.0 / sqrt_newton(sw / static_cast<double>(N) + eps);
+  }
+  __syncthreads();
+  const double r = rsh;
+  for (int64_t d0 = e0; d0 < e1; d0 += 256) {
+    const int64_t d = d0 + t;
+    const bool valid = d < N;
+    const double y = valid ? xf * r * wf : 0.0;
+    const int64_t nx = d + 256 < N ? d + 256 : N - 1;
+    xf = load_d<XDT>(X, base + nx);
+    wf = load_d<XDT>(W, nx);
+    if (valid) {
+      if (Y) store_out<0>(Y, ydt, base + d, y);
+      if (Y32) Y32[base + d] = static_cast<float>(y);
+    }
+    if (Xq) q8_store(static_cast<float>(y), valid, base + d, Xq, Xs);
+  }
+}
+
 template <int GDT>
 __global__ void __launch_bounds__(256) k_swiglu_q8(const void *__restrict__ G, const void *__restrict__ U,
                                                    void *__restrict__ H, int hdt, int8_t *__restrict__ Xq,
@@ -223,6 +280,27 @@ extern "C" int vybdq_rmsnorm_q8(uint64_t X, uint64_t W, uint64_t Y, uint64_t Y32
   auto *q = reinterpret_cast<int8_t *>(Xq);
   auto *d = reinterpret_cast<float *>(Xs);
   const int per = static_cast<int>((N + 255) / 256);
+  // Rows are split over workgroups while the grid stays under 512 (each split re-reads and re-sums the
+  // row; measured, float32 5120 columns: 1 row 14.8 -> 6.0 us with a SwiGLU launch beside it, 64 rows
+  // 15.9 -> 8.5 (8 parts; 20 parts 9.1), 512 rows 23.6 -> 23.1 unsplit, 40 in 20 parts). Outputs over the
+  // inputs need the row in registers before the first store, and float64 rows unsplit are faster that way
+  // (512 rows 23.2 us against 24.7): the one-workgroup kernel.
+  auto overlaps = [](uint64_t o, int64_t ob, uint64_t i, int64_t ib) {
+    return o && o < i + static_cast<uint64_t>(ib) && i < o + static_cast<uint64_t>(ob);
+  };
+  bool alias = false;
+  for (const auto &in : {std::pair<uint64_t, int64_t>{X, M * N * dt_size(x_dt)}, {W, N * dt_size(x_dt)}})
+    alias = alias || overlaps(Y, M * N * dt_size(y_dt), in.first, in.second) ||
+            overlaps(Y32, 4 * M * N, in.first, in.second) || overlaps(Xq, M * N, in.first, in.second) ||
+            overlaps(Xs, M * N / 8, in.first, in.second);
+  const int64_t chunks = (N + 255) / 256, want = M < 512 ? 512 / M : 1;
+  const int64_t E = (chunks + (want < chunks ? want : chunks) - 1) / (want < chunks ? want : chunks) * 256;
+  const unsigned parts = static_cast<unsigned>((N + E - 1) / E);
+  if (!alias && (parts > 1 || x_dt != VYBDQ_F64) && M < 65536) {
+    VYBDQ_DISPATCH_ANY(x_dt, XDT, hipLaunchKernelGGL((k_rms_q8_parts<XDT>), dim3(parts, static_cast<unsigned>(M)),
+                                                     dim3(256), 0, s, x, w, y, y_dt, y32, q, d, N, E, eps));
+    return check_launch("vybdq_rmsnorm_q8");
+  }
 #define L(C) VYBDQ_DISPATCH_ANY(x_dt, XDT, hipLaunchKernelGGL((k_rms_q8<XDT, C>), dim3(static_cast<unsigned>(M)), \
                                                                 dim3(256), 0, s, x, w, y, y_dt, y32, q, d, N, eps))
   if (per <= 4) { L(4); }
