@@ -337,9 +337,9 @@ int vybdq_exl3_gemm(uint64_t trellis, uint64_t suh, uint64_t svh, uint64_t X, ui
 int vybdq_gemm(int wtype, uint64_t W, uint64_t X, uint64_t Y, int64_t M, int64_t N, int64_t K, int x_dt,
                int y_dt, int64_t ldy, uint64_t RS, uint64_t stream);
 
-/* Workspace bytes vybdq_gemm_ws can use at (M, N, K) (q4_0, Q8_0, Q4_K, Q5_K from 64 rows; Q6_K,
-   IQ2_S from 96 rows): split-K partials and the fp16 copy of a bf16/f32 X; 0 when the shape does
-   not use the workspace. */
+/* Workspace bytes vybdq_gemm_ws can use at (M, N, K) (up to 64 rows, K % 256 == 0, N % 64 == 0: split-K
+   partials; q4_0, Q8_0, Q4_K, Q5_K from 64 rows, Q6_K, IQ2_S from 96 rows: split-K partials and the
+   fp16 copy of a bf16/f32 X); 0 when the shape does not use the workspace. */
 int64_t vybdq_gemm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
 
 /* vybdq_gemm with a caller workspace ws (256-byte aligned, ws_bytes, any contents; 0 = none). With
@@ -349,7 +349,9 @@ int64_t vybdq_gemm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
    from the unsplit vybdq_gemm); bf16/f32 X is converted to fp16 once into the workspace instead of
    once per output tile, each row scaled by the power of two that brings its largest |x| into
    [2^14, 2^15) (multiplied back into the row's outputs), so X of any magnitude neither overflows nor
-   flushes to zero. Calls that share a workspace must not overlap. The reference's gemm_q80
+   flushes to zero. Up to 64 rows (K % 256 == 0, N % 64 == 0, W 16-byte aligned) the call runs on weights
+   streamed past X in LDS, X scaled the same way per row and 256 k; Q4_K, Q5_K, Q6_K and IQ2_S weights
+   are not rounded to fp16 there. Calls that share a workspace must not overlap. The reference's gemm_q80
    has no workspace (native/tools/gen_rpf.py:58-62); this is the same GEMM for shapes whose
    tiles alone do not fill the GPU. */
 int vybdq_gemm_ws(int wtype, uint64_t W, uint64_t X, uint64_t Y, int64_t M, int64_t N, int64_t K, int x_dt,

@@ -1,0 +1,112 @@
+"""GPU parity of the GEMM at a few X rows (M <= 64 with a workspace: X resident in LDS, weights
+streamed past it) against the float64 oracle."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import iquants, kquants, matmul
+from tests.test_gpu_gguf import gate, to_dev, x_as
+from vybforge_amd import ops, synth
+from vybforge_amd._lib import call, lib
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [ops.GGML_Q4_0, ops.GGML_Q8_0, ops.GGML_Q4_K, ops.GGML_Q5_K, ops.GGML_Q6_K, ops.GGML_IQ2_S]
+# (M, N, K): one row and full row fragments; one super-block; tiles of 64, 128 and 256 weight rows;
+# odd super-block counts (Q6_K / IQ2_S rows at every 2-byte alignment within 16); K ranges split
+SHAPES = [(1, 64, 256), (9, 192, 768), (16, 256, 512), (17, 384, 1280), (32, 512, 2304), (33, 128, 5120),
+          (48, 640, 1024), (63, 320, 768), (64, 256, 17408)]
+
+
+def weights(ty, rng, N, K):
+    if ty == ops.GGML_Q4_0:
+        raw = synth.q4_0_weights(rng, N, K)
+        return raw, matmul.q4_0_matrix(raw, N, K)
+    if ty == ops.GGML_Q8_0:
+        raw = synth.q8_0_weights(rng, N, K)
+        return raw, matmul.q8_0_matrix(raw, N, K)
+    raw = synth.kquant_weights(rng, ty, N, K)
+    return raw, (iquants.matrix_iq2_s if ty == ops.GGML_IQ2_S else lambda r, n, k: kquants.matrix(ty, r, n, k))(raw, N, K)
+
+
+@pytest.mark.parametrize("ty", TYPES)
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_rows_gemm(dev, ty, M, N, K):
+    """Every type at the edges of tiles, row fragments and K ranges; the same call without a workspace (the
+    general tiles) agrees within the gate."""
+    rng = np.random.default_rng(ty * 1000 + M + N + K)
+    raw, w = weights(ty, rng, N, K)
+    xd, x64 = x_as(synth.activations(rng, (M, K)), ("bf16", "f16", "f32")[(M + ty) % 3], dev)
+    xd = xd.reshape(M, K)
+    Wd = to_dev(raw, dev)
+    ws = ops.GemmWorkspace([(M, N, K)], dev, ty)
+    assert ws.nbytes > 0
+    ref = matmul.gemm_rows_f64(x64.reshape(M, K), w)
+    assert matmul.rel_maxnorm(ops.gemm(ty, Wd, xd, N, K, workspace=ws).cpu().numpy(), ref) < matmul.TOL
+    assert matmul.rel_maxnorm(ops.gemm(ty, Wd, xd, N, K).cpu().numpy(), ref) < matmul.TOL
+
+
+@pytest.mark.parametrize("ty", TYPES)
+@pytest.mark.parametrize("plan", ["1,1", "2,3", "3,2", "9,1"])
+def test_rows_gemm_plans(dev, monkeypatch, ty, plan):
+    """Forced K ranges and workgroups per range: several tiles per workgroup (the LDS stages run on across
+    tiles), a ragged last range, one range; f64 output with a residual and a wider row stride."""
+    monkeypatch.setenv("VYBDQ_TUNING", "1")
+    monkeypatch.setenv("VYBDQ_ROWS_PLAN", plan)
+    M, N, K, ldy = 21, 896, 1792, 1000
+    rng = np.random.default_rng(ty + len(plan))
+    raw, w = weights(ty, rng, N, K)
+    x = synth.activations(rng, (M, K)).astype(np.float16)
+    rs = synth.activations(rng, (M, ldy)).astype(np.float64)
+    Wd, Xd, y = to_dev(raw, dev), to_dev(x, dev), to_dev(rs, dev)
+    ws = ops.GemmWorkspace([(M, N, K)], dev, ty)
+    call("vybdq_gemm_ws", ty, Wd.data_ptr(), Xd.data_ptr(), y.data_ptr(), M, N, K, ops.F16, ops._dt(torch.float64), ldy,
+         y.data_ptr(), ws.ptr, ws.nbytes, torch.cuda.current_stream().cuda_stream)
+    got = y.cpu().numpy()
+    assert matmul.rel_maxnorm(got[:, :N], matmul.gemm_rows_f64(x.astype(np.float64), w, rs[:, :N])) < matmul.TOL
+    np.testing.assert_array_equal(got[:, N:], rs[:, N:])
+
+
+@pytest.mark.parametrize("ty", TYPES)
+@pytest.mark.parametrize("xdt", ["f16", "bf16", "f32"])
+def test_rows_gemm_ranges(dev, ty, xdt):
+    """Rows of very different magnitude, an outlier channel, an all-zero row and blocks: every row against its
+    own largest output (the power-of-two scales of X are per row and super-block)."""
+    M, N, K = 13, 256, 768
+    rng = np.random.default_rng(ty + len(xdt))
+    raw, w = weights(ty, rng, N, K)
+    x = rng.standard_normal((M, K))
+    big = 6e4 if xdt == "f16" else 1e30
+    x *= np.array([1.0, big / 8, 1e-3, 1.0, 100.0, 1e-2, 1.0, 1.0, 0.0, 1.0, 1.0, 1.0, 10.0])[:, None]
+    x[3, 300] = big
+    x[6, 256:512] = 0
+    x[7] += 1000.0
+    xd, x64 = x_as(x.astype(np.float32), xdt, dev)
+    ws = ops.GemmWorkspace([(M, N, K)], dev, ty)
+    y = ops.gemm(ty, to_dev(raw, dev), xd.reshape(M, K), N, K, y_dtype=torch.float64, workspace=ws).cpu().numpy()
+    ref = matmul.gemm_rows_f64(x64.reshape(M, K), w)
+    assert not y[8].any()
+    for m in range(M):
+        if m != 8:
+            assert gate(y[m:m + 1], ref[m:m + 1], torch.float64) < matmul.TOL, m
+
+
+@pytest.mark.parametrize("ty", [ops.GGML_Q4_K, ops.GGML_Q6_K])
+def test_rows_gemm_falls_back(dev, ty):
+    """Weights at a 4-byte address and a workspace that is too small take the general tiles."""
+    M, N, K = 24, 256, 1024
+    rng = np.random.default_rng(ty)
+    raw, w = weights(ty, rng, N, K)
+    x = synth.activations(rng, (M, K)).astype(np.float16)
+    ref = matmul.gemm_rows_f64(x.astype(np.float64), w)
+    off = torch.zeros(raw.size + 4, dtype=torch.uint8, device=dev)
+    off[4:] = to_dev(raw, dev)
+    Wd, Xd = to_dev(raw, dev), to_dev(x, dev)
+    ws = ops.GemmWorkspace([(M, N, K)], dev, ty)
+    assert matmul.rel_maxnorm(ops.gemm(ty, off[4:], Xd, N, K, workspace=ws).cpu().numpy(), ref) < matmul.TOL
+    y = torch.empty((M, N), dtype=torch.float32, device=dev)
+    call("vybdq_gemm_ws", ty, Wd.data_ptr(), Xd.data_ptr(), y.data_ptr(), M, N, K, ops.F16, ops.F32, 0, 0, ws.ptr, 256,
+         torch.cuda.current_stream().cuda_stream)
+    assert matmul.rel_maxnorm(y.cpu().numpy(), ref) < matmul.TOL
+    assert lib.vybdq_gemm_workspace_size(ty, M, N, K) == ws.nbytes

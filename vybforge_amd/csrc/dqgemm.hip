@@ -38,6 +38,9 @@ int mmq_gemm(int wtype, const void *W, const void *X, int xdt, void *Y, int ydt,
              int64_t ldy, const void *RS, void *ws, int64_t ws_bytes, hipStream_t s);
 int64_t mmq_i8_workspace_size(int64_t M, int64_t N, int64_t K);
 // the super-block (Q4_K, Q5_K, Q6_K, IQ2_S) GEMM (kqgemm.hip)
+int64_t rows_mm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
+int rows_mm_gemm(int wtype, const void *W, const void *X, int xdt, void *Y, int ydt, int64_t M, int64_t N, int64_t K,
+                 int64_t ldy, const void *RS, void *ws, int64_t ws_bytes, hipStream_t s);
 int64_t kq2_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
 int kq2_gemm(int wtype, const void *W, const void *X, int xdt, void *Y, int ydt, int64_t M, int64_t N, int64_t K,
              int64_t ldy, const void *RS, void *ws, int64_t ws_bytes, hipStream_t s);
@@ -420,6 +423,11 @@ int dq_gemm_grouped(int wtype, bool swiglu, const uint8_t *W, const uint8_t *W2,
 
 using namespace vybdq;
 
+// rows up to which a call with a workspace runs on rows_mm.h. At 64 rows, with both workspaces: 17408 x 5120 q4_0
+// 38 us against 48 on the prefill tiles, Q8_0 46 / 52, Q4_K 38 / 52, Q5_K 41 / 57, Q6_K 47 / 75, IQ2_S 41 / 81;
+// 6144 x 2048 14 to 17 us against 23 to 28. Above, its row fragments no longer fit registers and LDS.
+constexpr int64_t kRowsMmMax = 64;
+
 static int gemm_check(int wtype, uint64_t W, uint64_t X, uint64_t Y, int64_t M, int64_t N, int64_t K, int x_dt,
                       int y_dt, int64_t ldy) {
   VYBDQ_REQUIRE(W && X && Y, VYBDQ_ERR_ARG, "null W, X or Y");
@@ -448,6 +456,7 @@ static int gemm_check(int wtype, uint64_t W, uint64_t X, uint64_t Y, int64_t M, 
 }
 
 extern "C" int64_t vybdq_gemm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
+  if (M >= 1 && M <= kRowsMmMax && N >= 64 && K >= 256) return rows_mm_workspace_size(wtype, M, N, K);
   if (wtype == 14 || wtype == 22) return M >= 1 && N >= 64 && K >= 256 ? kq2_workspace_size(wtype, M, N, K) : 0;
   if ((wtype != 2 && wtype != 8 && wtype != 12 && wtype != 13) || M < 64 || !mmq_supported(M, N, K)) return 0;
   return mmq_workspace_size(wtype, M, N, K);
@@ -460,6 +469,13 @@ extern "C" int vybdq_gemm_ws(int wtype, uint64_t W, uint64_t X, uint64_t Y, int6
   if (rc) return rc;
   VYBDQ_REQUIRE(ws == 0 || (ws & 255) == 0, VYBDQ_ERR_ALIGN, "workspace must be 256-byte aligned");
   VYBDQ_REQUIRE(ws_bytes >= 0, VYBDQ_ERR_WORKSPACE, "negative workspace size");
+  if (M <= kRowsMmMax && ws) {
+    const int r = rows_mm_gemm(wtype, reinterpret_cast<const void *>(W), reinterpret_cast<const void *>(X), x_dt,
+                               reinterpret_cast<void *>(Y), y_dt, M, N, K, ldy ? ldy : N,
+                               reinterpret_cast<const void *>(RS), reinterpret_cast<void *>(ws), ws_bytes,
+                               as_stream(stream));
+    if (r != 1) return r;
+  }
   // Q4_K / Q5_K: the register-operand body streams fp16 X, so bf16 / f32 X needs room for its
   // conversion
   const bool q4k_ok = (wtype == 12 || wtype == 13) && M >= 64 && K < (int64_t(1) << 22) && mmq_supported(M, N, K) &&

@@ -1,0 +1,188 @@
+// Host side of the GEMM at a few X rows (rows_mm.h): plan, dispatch and the split reduce.
+#include "rows_mm.h"
+
+#include <cstdio>
+#include <cstdlib>
+
+namespace vybdq {
+
+constexpr int kRowsMaxSplits = 40;  // K splits: above, the partials outweigh the weights
+
+// the float32 partials of a K split summed in split order and stored with the residual
+template <int ODT>
+__global__ void __launch_bounds__(256) k_rows_reduce(const RowsArgs a) {
+  const int64_t n4 = a.N / 4, total = a.M * n4, stride = static_cast<int64_t>(a.M) * a.N;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= total) return;
+  const int64_t row = i / n4, c = 4 * (i % n4);
+  const float *p = a.part + row * a.N + c;
+  f4 v = f4{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < a.splits; s0 += 8) {  // eight loads in flight, added in split order
+    f4 t[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = *reinterpret_cast<const f4 *>(p + (s0 + u < a.splits ? s0 + u : 0) * stride);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (s0 + u < a.splits) v = v + t[u];
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) store_elem<ODT>(a.Y, a.RS, row * a.ldy + c + u, v[u]);
+}
+
+struct RowsPlan {
+  int NW, splits, sps, nwg, ns;  // waves (16 weight rows each), K splits, super-blocks per split, workgroups per split, stages
+};
+
+// 16 waves (256 weight rows a tile) up to 32 X rows: with 8 (two per SIMD) a wave's decode waits on its
+// own LDS reads and matrix-core chains (Q4_K 17408 x 5120, 24 rows: 25.2 us against 26.9). Above, the accumulators
+// need the registers of 8 waves; and so may LDS (Q8_0: two stages of 256 rows and one X super-block are all
+// of it). One workgroup fits a CU; the plan minimises the stages of the busiest CU (a stage's bytes at
+// the 18.5 GB/s a CU gets of HBM) plus a workgroup's start (X staging) and the split partials, written
+// and read back. With only two LDS stages a stage is barely in flight: 10% more. VYBDQ_ROWS_PLAN="sps,nwg"
+// overrides the split (ignored where it does not fit).
+template <int FMT>
+static RowsPlan rows_plan(int M, int64_t N, int64_t K, bool split) {
+  using F = RowsFmt<FMT>;
+  const int SB = static_cast<int>(K / 256), MF = (M + 15) / 16, cus = 256;
+  const int xsb = MF * (F::OPS * 1024 + 64), tab = FMT == FMT_IQ2_S ? kRowsGrid : 0;
+  RowsPlan best{};
+  double best_t = -1;
+  int fs = 0, fn = 0;
+  if (const char *e = tuning_env("VYBDQ_ROWS_PLAN"))
+    if (sscanf(e, "%d,%d", &fs, &fn) != 2 || fs < 1 || fn < 1) fs = fn = 0;
+  for (int NW = MF <= 2 ? 16 : 8; NW >= 4; NW /= 2) {
+    const int BN = 16 * NW, tiles = static_cast<int>(N / BN), stage = BN * F::C * 16;
+    if (N % BN || (NW == 4 && N % 128 == 0)) continue;  // 4 waves only where 8 do not divide N
+    for (int sps = 1; sps <= SB && sps <= 32; ++sps) {
+      const int splits = (SB + sps - 1) / sps;
+      int ns = (160 * 1024 - tab - sps * xsb) / stage;
+      if (ns < 2) break;
+      ns = ns > 4 ? 4 : ns;
+      if (splits > (split ? kRowsMaxSplits : 1)) continue;
+      int nwg = cus / splits > 0 ? cus / splits : 1;
+      if (fs) {
+        if (sps != (fs < SB ? fs : SB)) continue;
+        nwg = fn;
+      }
+      nwg = nwg < tiles ? nwg : tiles;
+      const int rounds = (splits * nwg + cus - 1) / cus, stages = (tiles + nwg - 1) / nwg * sps;
+      double t = rounds * (stages * stage / 18.5e3 * (ns == 2 ? 1.1 : 1.0) + 2.5 + 0.2 * sps * MF);
+      if (NW < 16 && MF <= 2) t *= 1.08;
+      if (splits > 1) t += 4.0 + 8.0 * splits * M * static_cast<double>(N) / 4.0e6;
+      if (best_t < 0 || t < best_t) {
+        best_t = t;
+        best = {NW, splits, sps, nwg, ns};
+      }
+    }
+  }
+  return best;  // splits = 0: no plan fits
+}
+
+bool rows_mm_supported(int wtype, int64_t M, int64_t N, int64_t K) {
+  return M >= 1 && M <= 64 && K % 256 == 0 && K < (int64_t(1) << 22) && N % 64 == 0 &&
+         (wtype == 2 || wtype == 8 || wtype == 12 || wtype == 13 || wtype == 14 || wtype == 22);
+}
+
+// the plan of a type id
+static RowsPlan rows_plan_ty(int wtype, int M, int64_t N, int64_t K, bool split) {
+  switch (wtype) {
+    case 2: return rows_plan<FMT_Q4_0>(M, N, K, split);
+    case 8: return rows_plan<FMT_Q8_0>(M, N, K, split);
+    case 12: return rows_plan<FMT_Q4_K>(M, N, K, split);
+    case 13: return rows_plan<FMT_Q5_K>(M, N, K, split);
+    case 14: return rows_plan<FMT_Q6_K>(M, N, K, split);
+    default: return rows_plan<FMT_IQ2_S>(M, N, K, split);
+  }
+}
+
+// workspace: split partials (at least 256 bytes where the shape is taken, so that a caller has one)
+int64_t rows_mm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
+  if (!rows_mm_supported(wtype, M, N, K)) return 0;
+  const RowsPlan p = rows_plan_ty(wtype, static_cast<int>(M), N, K, true);
+  if (p.splits == 0) return 0;
+  return p.splits > 1 ? static_cast<int64_t>(p.splits) * M * N * 4 : 256;
+}
+
+template <int FMT, int XDT, int MF, int NW>
+static int rows_launch(const RowsArgs &a, const RowsPlan &p, hipStream_t s) {
+  using Sh = RowsShape<FMT, MF, NW>;
+  static std::atomic<uint64_t> raised{0};
+  const int rc = ensure_lds_limit(reinterpret_cast<const void *>(&k_rows_mm<FMT, XDT, MF, NW>), 160 * 1024, raised,
+                                  "gemm (few rows)");
+  if (rc) return rc;
+  const size_t lds = Sh::TAB + static_cast<size_t>(p.sps) * Sh::XSB + static_cast<size_t>(p.ns) * Sh::STAGE;
+  hipLaunchKernelGGL((k_rows_mm<FMT, XDT, MF, NW>), dim3(static_cast<unsigned>(p.nwg), static_cast<unsigned>(p.splits)),
+                     dim3(64 * NW), lds, s, a);
+  return check_launch("gemm (few rows)");
+}
+
+template <int FMT, int XDT, int MF>
+static int rows_launch_p(const RowsArgs &a, const RowsPlan &p, hipStream_t s) {
+  if constexpr (MF <= 2) {
+    if (p.NW == 16) return rows_launch<FMT, XDT, MF, 16>(a, p, s);
+  }
+  if (p.NW == 8) return rows_launch<FMT, XDT, MF, 8>(a, p, s);
+  return rows_launch<FMT, XDT, MF, 4>(a, p, s);
+}
+
+template <int FMT, int XDT>
+static int rows_launch_x(const RowsArgs &a, const RowsPlan &p, hipStream_t s) {
+  switch ((a.M + 15) / 16) {
+    case 1: return rows_launch_p<FMT, XDT, 1>(a, p, s);
+    case 2: return rows_launch_p<FMT, XDT, 2>(a, p, s);
+    case 3: return rows_launch_p<FMT, XDT, 3>(a, p, s);
+    default: return rows_launch_p<FMT, XDT, 4>(a, p, s);
+  }
+}
+
+template <int FMT>
+static int rows_run_fmt(RowsArgs &a, int xdt, void *ws, int64_t ws_bytes, hipStream_t s) {
+  const int64_t K = static_cast<int64_t>(a.SB) * 256;
+  const RowsPlan p = rows_plan<FMT>(a.M, a.N, K, ws != nullptr);
+  if (p.splits == 0 || (p.splits > 1 && ws_bytes < static_cast<int64_t>(p.splits) * a.M * a.N * 4)) return 1;
+  a.rowbytes = unit_row_bytes<FMT>(K / 64);
+  a.splits = p.splits;
+  a.sps = p.sps;
+  a.ns = p.ns;
+  a.tiles = a.N / (16 * p.NW);
+  a.part = static_cast<float *>(ws);
+#ifdef ROWS_PROBE
+  if (xdt != VYBDQ_BF16) return 1;
+  return rows_launch_x<FMT, VYBDQ_BF16>(a, p, s);
+#else
+  int rc = VYBDQ_OK;
+  VYBDQ_DISPATCH_IN(xdt, XDT, rc = rows_launch_x<FMT, XDT>(a, p, s));
+  return rc;
+#endif
+}
+
+// Returns 1 when the call does not fit (shape, W not 16-byte aligned).
+int rows_mm_gemm(int wtype, const void *W, const void *X, int xdt, void *Y, int ydt, int64_t M, int64_t N, int64_t K,
+                 int64_t ldy, const void *RS, void *ws, int64_t ws_bytes, hipStream_t s) {
+  if (!rows_mm_supported(wtype, M, N, K) || (reinterpret_cast<uintptr_t>(W) & 15)) return 1;
+  RowsArgs a{};
+  a.W = static_cast<const uint8_t *>(W);
+  a.X = X;
+  a.M = static_cast<int>(M);
+  a.N = static_cast<int>(N);
+  a.SB = static_cast<int>(K / 256);
+  a.Y = Y;
+  a.ydt = ydt;
+  a.ldy = ldy;
+  a.RS = RS;
+  int rc;
+  switch (wtype) {
+    case 2: rc = rows_run_fmt<FMT_Q4_0>(a, xdt, ws, ws_bytes, s); break;
+    case 8: rc = rows_run_fmt<FMT_Q8_0>(a, xdt, ws, ws_bytes, s); break;
+    case 12: rc = rows_run_fmt<FMT_Q4_K>(a, xdt, ws, ws_bytes, s); break;
+    case 13: rc = rows_run_fmt<FMT_Q5_K>(a, xdt, ws, ws_bytes, s); break;
+    case 14: rc = rows_run_fmt<FMT_Q6_K>(a, xdt, ws, ws_bytes, s); break;
+    default: rc = rows_run_fmt<FMT_IQ2_S>(a, xdt, ws, ws_bytes, s); break;
+  }
+  if (rc || a.splits == 1) return rc;
+  const unsigned grid = static_cast<unsigned>((M * N / 4 + 255) / 256);
+  VYBDQ_DISPATCH_OUT(ydt, ODT, hipLaunchKernelGGL((k_rows_reduce<ODT>), dim3(grid), dim3(256), 0, s, a));
+  return check_launch("gemm (few rows) split reduce");
+}
+
+}  // namespace vybdq
