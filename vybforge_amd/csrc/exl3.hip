@@ -116,8 +116,8 @@ __global__ void __launch_bounds__(256) k_exl3_dequant(const uint16_t *__restrict
 //    operands, every batch size), the waves' partials summed in LDS in a fixed order. Bound by the
 //    hash on the VALU (4.0 instructions per weight, 80% of the issue slots while it runs) and, at one row,
 //    by ~8 us per call that do not scale with K (x rotation, arrival, output rotation). K = 5120,
-//    N = 17408: batch 16 23.2 us (29.2 with the decoded words regrouped through LDS, 7.3
-//    instructions per weight), batch 1 20.0 (20.5 with one dot product per weight and lane, 5.0).
+//    N = 17408: batch 16 23 us (29.2 with the decoded words regrouped through LDS, 7.3
+//    instructions per weight), batch 1 19.3 (20.5 with one dot product per weight and lane, 5.0).
 // 3. y[b][n] = svh[n] * FWHT(sum_s z_s[b][.]) / sqrt(128), sums in split order. Batch <= 2: the
 //    last split of a column block to arrive (a per-block arrival counter, reset by that last
 //    arrival so the counters stay zero between calls) does it; larger batches: k_exl3_out.
@@ -140,7 +140,7 @@ __global__ void __launch_bounds__(64) k_exl3_xprep(const void *__restrict__ X, c
 }
 
 template <bool FUSED>
-__global__ void __launch_bounds__(256, 4) k_exl3_gemm(const uint16_t *__restrict__ trellis, const void *__restrict__ X,
+__global__ void __launch_bounds__(256, 5) k_exl3_gemm(const uint16_t *__restrict__ trellis, const void *__restrict__ X,
                                                       int xdt, const _Float16 *__restrict__ suh,
                                                       const _Float16 *__restrict__ svh, void *__restrict__ Y, int ydt,
                                                       int B, int BP, const _Float16 *__restrict__ xp,

@@ -148,10 +148,10 @@ __device__ __forceinline__ void exl3_barrier() {
 // step whole 1 KB runs. `base`: the first step's first tile (wave-uniform); `kstride`: uint16 from
 // one k-block to the next; aload(st, v): step st's 16 x' values (k-block l >> 4 of the step) of row
 // l & 15 (any finite or other values for rows past the group: they reach only outputs that are not
-// stored), two steps ahead if AHEAD (x' in memory) or at the step (x' in LDS); ready() runs between the first trellis loads and the first aload (it may stage x' in LDS and
-// wait for it: the trellis loads stay in flight across an exl3_barrier). acc[2 c + h][r] = z[row 4 (l >> 4) + r][exl3_mma_col(c, h, l)]. Two steps of loads are in
-// flight per lane (8 KB per wave); each ring slot is refilled right after its use, pinned by
-// scheduling barriers (sunk to the end of the step it would leave no load in flight).
+// stored), a step ahead if AHEAD (x' in memory) or at the step (x' in LDS); ready() runs between the first trellis loads and the first aload (it may stage x' in LDS and
+// wait for it: the trellis loads stay in flight across an exl3_barrier). acc[2 c + h][r] = z[row 4 (l >> 4) + r][exl3_mma_col(c, h, l)]. A step of loads (4 KB per
+// wave) is in flight per lane; each ring slot is refilled right after its use, pinned by scheduling
+// barriers (sunk to the end of the step it would leave no load in flight).
 template <bool AHEAD, class Ready, class ALoad>
 __device__ __forceinline__ void exl3_mma_run(const uint16_t *__restrict__ base, int64_t kstride, int nsteps,
                                              const Ready &ready, const ALoad &aload, f4 (&acc)[8]) {
@@ -161,7 +161,7 @@ __device__ __forceinline__ void exl3_mma_run(const uint16_t *__restrict__ base, 
   }
   const int lane = threadIdx.x & 63, n = lane & 15;
   const uint16_t *lp = base + (lane >> 4) * kstride + 8 * n;
-  constexpr int R = 2;
+  constexpr int R = 1;  // two steps ahead (114 VGPRs, four waves per SIMD instead of five) measured 3% slower
   u4 ring[R][4], xr[AHEAD ? R : 1][2];
   auto wload = [&](int st, int c) {
     const int sc = st < nsteps ? st : nsteps - 1;  // in range: re-read the last

@@ -314,14 +314,14 @@ struct MxGemmArgs {
 // partials summed in LDS in a fixed order. The group index is the fastest grid dimension and the
 // bound is a multiple of 8, so every column block of one group runs on the same XCD (its L2 holds
 // the group's x' rows). Bound by the hash on the VALU (4.0 instructions per weight, 82% of the issue
-// slots). 256 tokens, H = 4096, I = 2048, 288 experts: gate | up 735 us, down 426 us (995 and 563 with the
+// slots). 256 tokens, H = 4096, I = 2048, 288 experts: gate | up 690 us, down 395 us (995 and 563 with the
 // decoded words regrouped through LDS, 7.3 instructions per weight).
 // SH: the launch also carries the shared expert's tiles (0 none; 1 gate | up, bf16 activations;
 // 2 gate | up, activations as bf16 hi + lo terms; 3 down, hi + lo), as workgroups with blockIdx.y
 // past the routed column blocks: its bf16 weights stream from HBM while the routed workgroups
 // decode trellis on the VALU.
 template <int SH>
-__global__ void __launch_bounds__(256, 4) k_mx_gemm(const MxGemmArgs a, const MxShared sh) {
+__global__ void __launch_bounds__(256, 5) k_mx_gemm(const MxGemmArgs a, const MxShared sh) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int jt = blockIdx.x;
   if constexpr (SH != 0) {
