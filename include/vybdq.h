@@ -339,7 +339,8 @@ int vybdq_gemm(int wtype, uint64_t W, uint64_t X, uint64_t Y, int64_t M, int64_t
 
 /* Workspace bytes vybdq_gemm_ws can use at (M, N, K) (up to 64 rows, K % 256 == 0, N % 64 == 0: split-K
    partials; q4_0, Q8_0, Q4_K, Q5_K from 64 rows, Q6_K, IQ2_S from 96 rows: split-K partials and the
-   fp16 copy of a bf16/f32 X); 0 when the shape does not use the workspace. */
+   fp16 copy of a bf16/f32 X; long prompts of large matrices: 2 N K bytes more, the fp16 weights); 0 when
+   the shape does not use the workspace. */
 int64_t vybdq_gemm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
 
 /* vybdq_gemm with a caller workspace ws (256-byte aligned, ws_bytes, any contents; 0 = none). With
@@ -351,7 +352,9 @@ int64_t vybdq_gemm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
    [2^14, 2^15) (multiplied back into the row's outputs), so X of any magnitude neither overflows nor
    flushes to zero. Up to 64 rows (K % 256 == 0, N % 64 == 0, W 16-byte aligned) the call runs on weights
    streamed past X in LDS, X scaled the same way per row and 256 k; Q4_K, Q5_K, Q6_K and IQ2_S weights
-   are not rounded to fp16 there. Calls that share a workspace must not overlap. The reference's gemm_q80
+   are not rounded to fp16 there. Long prompts of large matrices (the size tells: 2 N K bytes more) expand
+   W to fp16 in the workspace once and run a plain fp16 tile GEMM over it; a smaller workspace keeps the
+   fused bodies. Calls that share a workspace must not overlap. The reference's gemm_q80
    has no workspace (native/tools/gen_rpf.py:58-62); this is the same GEMM for shapes whose
    tiles alone do not fill the GPU. */
 int vybdq_gemm_ws(int wtype, uint64_t W, uint64_t X, uint64_t Y, int64_t M, int64_t N, int64_t K, int x_dt,

@@ -41,6 +41,9 @@ int64_t mmq_i8_workspace_size(int64_t M, int64_t N, int64_t K);
 int64_t rows_mm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
 int rows_mm_gemm(int wtype, const void *W, const void *X, int xdt, void *Y, int ydt, int64_t M, int64_t N, int64_t K,
                  int64_t ldy, const void *RS, void *ws, int64_t ws_bytes, hipStream_t s);
+int64_t wide_mm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
+int wide_mm_gemm(int wtype, const void *W, const void *X, int xdt, void *Y, int ydt, int64_t M, int64_t N, int64_t K,
+                 int64_t ldy, const void *RS, void *ws, int64_t ws_bytes, hipStream_t s);
 int64_t kq2_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
 int kq2_gemm(int wtype, const void *W, const void *X, int xdt, void *Y, int ydt, int64_t M, int64_t N, int64_t K,
              int64_t ldy, const void *RS, void *ws, int64_t ws_bytes, hipStream_t s);
@@ -455,11 +458,18 @@ static int gemm_check(int wtype, uint64_t W, uint64_t X, uint64_t Y, int64_t M, 
   return VYBDQ_OK;
 }
 
-extern "C" int64_t vybdq_gemm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
+// what the fused bodies use (0: nothing)
+static int64_t fused_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
   if (M >= 1 && M <= kRowsMmMax && N >= 64 && K >= 256) return rows_mm_workspace_size(wtype, M, N, K);
   if (wtype == 14 || wtype == 22) return M >= 1 && N >= 64 && K >= 256 ? kq2_workspace_size(wtype, M, N, K) : 0;
   if ((wtype != 2 && wtype != 8 && wtype != 12 && wtype != 13) || M < 64 || !mmq_supported(M, N, K)) return 0;
   return mmq_workspace_size(wtype, M, N, K);
+}
+
+extern "C" int64_t vybdq_gemm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
+  const int64_t fused = fused_workspace_size(wtype, M, N, K);
+  const int64_t wide = M >= 1 && N >= 64 && K >= 256 ? wide_mm_workspace_size(wtype, M, N, K) : 0;
+  return wide > fused ? wide : fused;
 }
 
 extern "C" int vybdq_gemm_ws(int wtype, uint64_t W, uint64_t X, uint64_t Y, int64_t M, int64_t N, int64_t K,
@@ -471,6 +481,13 @@ extern "C" int vybdq_gemm_ws(int wtype, uint64_t W, uint64_t X, uint64_t Y, int6
   VYBDQ_REQUIRE(ws_bytes >= 0, VYBDQ_ERR_WORKSPACE, "negative workspace size");
   if (M <= kRowsMmMax && ws) {
     const int r = rows_mm_gemm(wtype, reinterpret_cast<const void *>(W), reinterpret_cast<const void *>(X), x_dt,
+                               reinterpret_cast<void *>(Y), y_dt, M, N, K, ldy ? ldy : N,
+                               reinterpret_cast<const void *>(RS), reinterpret_cast<void *>(ws), ws_bytes,
+                               as_stream(stream));
+    if (r != 1) return r;
+  }
+  if (M > kRowsMmMax && ws) {
+    const int r = wide_mm_gemm(wtype, reinterpret_cast<const void *>(W), reinterpret_cast<const void *>(X), x_dt,
                                reinterpret_cast<void *>(Y), y_dt, M, N, K, ldy ? ldy : N,
                                reinterpret_cast<const void *>(RS), reinterpret_cast<void *>(ws), ws_bytes,
                                as_stream(stream));
