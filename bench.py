@@ -948,7 +948,7 @@ def run_moe_exl3(args, torch, dev, tokens=None, built=None):
         rel = check_moe_exl3(torch, layers[r], xs[r], lgs[r], outs[r], routed[r][1], routed[r][2])
         check = dict(ok=True, rel=rel, what="routing of every token; the last token x 256 columns vs float64 "
                                             "oracle; graph replay == eager")
-    gemm = "k_mx_gemm<1>" if T == 1 else ("k_mx_gemm<2>" if T * k <= 2 * min(E, T * k) else "k_mx_gemm<16>")
+    gemm = f"k_mx_gemm (groups of {1 if T == 1 else 16} rows)"
     roofline = hbm_roofline(gbs, f"EXL3 MoE layer: route+bucket, x rotation, {gemm} gate|up and down (trellis "
                                  "decoded in registers), SwiGLU between rotations, bf16 shared expert, combine",
                             "algorithmic bytes (hit experts' trellis + scales, shared expert, activations) / "
