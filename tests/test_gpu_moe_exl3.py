@@ -131,6 +131,35 @@ def test_moe_exl3_combine_chunks(dev, monkeypatch, T):
     np.testing.assert_array_equal(ys[0], ys[1])
 
 
+@pytest.mark.parametrize("E,k,H,ldt,with_bias", [
+    (1, 1, 128, "f32", True), (64, 64, 128, "bf16", False), (320, 8, 640, "f64", True), (321, 9, 1280, "f16", True),
+    (1024, 64, 128, "bf16", True), (288, 8, 4224, "f32", False)])
+def test_moe_exl3_one_token_routing(dev, E, k, H, ldt, with_bias):
+    """One token: routed, grouped and rotated in one launch, at the edges of its experts per lane (320 / 321,
+    1024), slots (1, 64), chunks per wave (1, 2, 5) and logit types (bf16: ties go to the lower id), with
+    the experts drawn from a pool of five; the routing exactly, outputs against the oracle."""
+    I, P = 128, 5
+    rng = np.random.default_rng(E + k)
+    host = [_expert_tensors(rng, H, I) for _ in range(P)]
+    pool = [_to_dev(h, dev) for h in host]
+    bias = rng.standard_normal(E).astype(np.float32) * 0.1 if with_bias else None
+    layer = ops.MoeExl3Layer([pool[e % P] for e in range(E)], H, I, topk=k,
+                             bias=torch.from_numpy(bias).to(dev) if with_bias else None)
+    x = _x(rng, 1, H, "bf16")
+    dt = {"f64": torch.float64, "f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[ldt]
+    logits = torch.from_numpy(rng.standard_normal((1, E))).to(dt)
+    cache = {e: tuple(exl3.dequant_exl3_f64(host[e][3 * p], host[e][3 * p + 1], host[e][3 * p + 2]).T
+                      for p in range(3)) for e in range(P)}
+    zero = (np.zeros((I, H)), np.zeros((I, H)), np.zeros((H, I)))
+    ref, ridx, rw = moe.moe_forward(x.to(torch.float64).numpy(), logits.to(torch.float64).numpy(),
+                                    lambda e: cache[e % P], zero, topk=k, bias=bias)
+    for _ in range(3):  # the second and third call find the first one's routing in the workspace
+        y, idx, w = layer(x.to(dev), logits.to(dev), routing=True)
+        np.testing.assert_array_equal(idx.cpu().numpy(), ridx)
+        assert np.abs(w.cpu().numpy() - rw).max() < 1e-6
+        assert matmul.rel_maxnorm(y.cpu().numpy(), ref) < TOL
+
+
 def test_moe_exl3_out_dtypes_and_f16_x(dev):
     """fp16 activations (two bf16 terms into the shared expert) and bf16 / fp16 outputs."""
     H, I, E, k, T = 256, 128, 6, 2, 9

@@ -12,6 +12,7 @@
 // weight (x W = svh * FWHT(FWHT(x * suh)/sqrt(128) What)/sqrt(128) per 128 chunk):
 //  1. route + bucket (moe.hip): rows = (token, slot) pairs grouped by expert; groups of at most 16
 //     rows of one expert (of one row at one token).
+//     One token: 1 and 2 are one launch (k_mx_route_xprep).
 //  2. k_mx_xprep: x'[p][row] = FWHT(x[token] * suh_{e,p}) / sqrt(128), p = gate, up, stored as fp16
 //     after a power-of-two scale per row that brings its largest |x'| into [2^14, 2^15) (exact;
 //     multiplied back after the product, which is linear in x'): no overflow, no fp16 subnormals.
@@ -36,6 +37,7 @@
 // glm_engine.vyb:2845-2862). Trellis int16 [in/16][out/16][64], 16-byte aligned; suh fp16 [in],
 // svh fp16 [out]; codebook mcg (the only one the reference has).
 #include "exl3_dev.h"
+#include "moe_route.h"
 
 namespace vybdq {
 
@@ -115,29 +117,21 @@ __device__ __forceinline__ float mx_row_max(float v, float *wm) {
   return m;
 }
 
-template <int XDT, int CPW>
-__global__ void __launch_bounds__(64 * kMxRowWaves) k_mx_xprep(const void *__restrict__ X,
-                                                              const uint64_t *__restrict__ tab,
-                                                              const int *__restrict__ idx, const int *__restrict__ pos,
-                                                              int topk, int64_t H, int rows, _Float16 *__restrict__ xp,
-                                                              float *__restrict__ xscale) {
-  __shared__ float wm[kMxRowWaves];
-  const int i = blockIdx.x, p = blockIdx.y, lane = threadIdx.x & 63;
+// The rotation of one row for projection p: chunk c of the row is wave c mod 8's, x holds its elements.
+template <int CPW>
+__device__ __forceinline__ void mx_rotate_row(float (&a)[CPW][2], const _Float16 *suh, int p, int r, int64_t H, int rows,
+                                              _Float16 *__restrict__ xp, float *__restrict__ xscale, float *wm) {
+  const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int64_t t = i / topk;
-  const int e = idx[i], r = pos[i];
-  const _Float16 *suh = mx_ptr<_Float16>(tab, e, p, 1);
   const int nch = static_cast<int>(H / 128);
-  float a[CPW][2];
   float amax = 0.f;
 #pragma unroll
   for (int q = 0; q < CPW; ++q) {
     const int c = wave + kMxRowWaves * q;
-    a[q][0] = a[q][1] = 0.f;
     if (c < nch) {
       const int64_t k0 = 128 * static_cast<int64_t>(c) + 2 * lane;
-      a[q][0] = load_elem<XDT>(X, t * H + k0) * static_cast<float>(suh[k0]);
-      a[q][1] = load_elem<XDT>(X, t * H + k0 + 1) * static_cast<float>(suh[k0 + 1]);
+      a[q][0] *= static_cast<float>(suh[k0]);
+      a[q][1] *= static_cast<float>(suh[k0 + 1]);
       fwht128_wave(a[q][0], a[q][1]);
       amax = fmaxf(amax, fmaxf(fabsf(a[q][0]), fabsf(a[q][1])));
     }
@@ -153,6 +147,93 @@ __global__ void __launch_bounds__(64 * kMxRowWaves) k_mx_xprep(const void *__res
           h2{static_cast<_Float16>(a[q][0] * f), static_cast<_Float16>(a[q][1] * f)};
   }
   if (threadIdx.x == 0) xscale[p * rows + r] = sc;
+}
+
+// x elements of token t, the chunks of mx_rotate_row
+template <int XDT, int CPW>
+__device__ __forceinline__ void mx_load_row(const void *__restrict__ X, int64_t t, int64_t H, float (&a)[CPW][2]) {
+  const int lane = threadIdx.x & 63, nch = static_cast<int>(H / 128);
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+#pragma unroll
+  for (int q = 0; q < CPW; ++q) {
+    const int c = wave + kMxRowWaves * q;
+    a[q][0] = a[q][1] = 0.f;
+    if (c < nch) {
+      const int64_t k0 = 128 * static_cast<int64_t>(c) + 2 * lane;
+      a[q][0] = load_elem<XDT>(X, t * H + k0);
+      a[q][1] = load_elem<XDT>(X, t * H + k0 + 1);
+    }
+  }
+}
+
+// One token: its routing, its rows' groups and their rotations in one launch. Workgroup (slot, p) repeats
+// the routing for itself (route_wg_keys / route_wg_select: the same keys, selection and weights as the launch
+// of its own) with its x elements already in flight, and rotates that slot's row; workgroup (topk, 0) writes
+// the routing outputs and the groups. Both parts are latency: 6.3 us + 5.0 us and the gap between them as two launches, 9.1 us as one (288
+// experts, H = 4096: layer 69.0 -> 66.7 us, in a graph 60 -> 57.4; 1024 experts 37.3 -> 33.9; 64 slots 88.8 -> 81.8). Only
+// at one token: with more, a row's place depends on every token's routing.
+template <int XDT, int CPW, int ENT>
+__global__ void __launch_bounds__(64 * kMxRowWaves) k_mx_route_xprep(
+    const void *__restrict__ X, const uint64_t *__restrict__ tab, const void *__restrict__ logits, int ldt,
+    const float *__restrict__ bias, int E, int topk, double scale, int64_t H, int *__restrict__ idx_out,
+    float *__restrict__ w_out, int *__restrict__ pos, int *__restrict__ row_map, int4 *__restrict__ tiles,
+    int *__restrict__ ntiles, int4 *__restrict__ groups, int *__restrict__ ngroups, _Float16 *__restrict__ xp,
+    float *__restrict__ xscale) {
+  __shared__ float wm[kMxRowWaves];
+  __shared__ int idx_lds[64];
+  __shared__ uint64_t key_lds[64 * ENT];
+  __shared__ double score_lds[64 * ENT];
+  const int i = blockIdx.x, p = blockIdx.y;
+  const bool writer = i == topk;  // the whole workgroup
+  if (writer && p) return;
+  float a[CPW][2];
+  if (!writer) mx_load_row<XDT, CPW>(X, 0, H, a);
+  switch (ldt) {
+    case VYBDQ_F64: route_wg_keys<VYBDQ_F64>(logits, bias, 0, E, key_lds, score_lds); break;
+    case VYBDQ_F32: route_wg_keys<VYBDQ_F32>(logits, bias, 0, E, key_lds, score_lds); break;
+    case VYBDQ_F16: route_wg_keys<VYBDQ_F16>(logits, bias, 0, E, key_lds, score_lds); break;
+    default: route_wg_keys<VYBDQ_BF16>(logits, bias, 0, E, key_lds, score_lds); break;
+  }
+  __syncthreads();
+  if (writer) {
+    if (threadIdx.x < 64) {
+      route_wg_select<ENT>(0, E, topk, scale, idx_out, w_out, idx_lds, key_lds, score_lds);
+      // one wave: its LDS stores above are in order before these reads
+      bucket_rows_wave(idx_lds, 1, topk, 1, 1, 0, pos, row_map, tiles, ntiles, groups, ngroups);
+    }
+    return;
+  }
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    uint64_t key[ENT];
+    uint32_t eid[ENT];
+#pragma unroll
+    for (int j = 0; j < ENT; ++j) {
+      const int e = lane + 64 * j;
+      key[j] = e < E ? key_lds[e] : 0;
+      eid[j] = e < E ? static_cast<uint32_t>(e) : kRouteNone;
+    }
+    const uint32_t mine = route_select<ENT>(key, eid, topk);
+    if (lane < topk) idx_lds[lane] = static_cast<int>(mine);
+  }
+  __syncthreads();
+  const int e = __builtin_amdgcn_readfirstlane(idx_lds[i]);
+  int r = 0;  // the row: a token's experts are distinct, rows are in expert order
+  for (int j = 0; j < topk; ++j) r += idx_lds[j] < e;
+  mx_rotate_row<CPW>(a, mx_ptr<_Float16>(tab, e, p, 1), p, __builtin_amdgcn_readfirstlane(r), H, topk, xp, xscale, wm);
+}
+
+template <int XDT, int CPW>
+__global__ void __launch_bounds__(64 * kMxRowWaves) k_mx_xprep(const void *__restrict__ X,
+                                                              const uint64_t *__restrict__ tab,
+                                                              const int *__restrict__ idx, const int *__restrict__ pos,
+                                                              int topk, int64_t H, int rows, _Float16 *__restrict__ xp,
+                                                              float *__restrict__ xscale) {
+  __shared__ float wm[kMxRowWaves];
+  const int i = blockIdx.x, p = blockIdx.y;
+  float a[CPW][2];
+  mx_load_row<XDT, CPW>(X, i / topk, H, a);
+  mx_rotate_row<CPW>(a, mx_ptr<_Float16>(tab, idx[i], p, 1), p, pos[i], H, rows, xp, xscale, wm);
 }
 
 // ---- 6. shared expert: bf16 weights on the matrix cores, carried by the routed launches ----------
@@ -695,22 +776,46 @@ extern "C" int vybdq_moe_forward_exl3(uint64_t x, int x_dt, uint64_t logits, int
   const int n = static_cast<int>(T * topk), k = static_cast<int>(topk);
 
   // 1. routing and row groups of at most BP rows
-  int rc = moe_route_bucket(reinterpret_cast<const void *>(logits), logits_dt, reinterpret_cast<const float *>(bias),
-                            T, E, topk, scale, p.BP, idx, wts, m.pos, m.row_map, m.tiles, m.ntiles, m.groups,
-                            m.ngroups, s);
-  if (rc) return rc;
   // 2. x' rows for gate and up
   const int cpw_h = static_cast<int>((H / 128 + kMxRowWaves - 1) / kMxRowWaves);
   const int cpw_i = static_cast<int>((I / 128 + kMxRowWaves - 1) / kMxRowWaves);
+  const int64_t lbytes = E * (logits_dt == VYBDQ_F64 ? 8 : logits_dt == VYBDQ_F32 ? 4 : 2);
+  auto apart = [&](uint64_t o) {  // routing outputs off everything the one launch's workgroups read
+    const auto off = [&](uint64_t i, int64_t ib) { return o + 4 * topk <= i || i + ib <= o; };
+    return !o || (off(logits, lbytes) && (!bias || off(bias, 4 * E)) && off(x, H * dt_size(x_dt)) && off(experts, 8 * kMxTab * E));
+  };
+  int rc;
+  if (T == 1 && apart(idx_out) && apart(w_out)) {
+#define RXE(XDT, CPW, ENT)                                                                                       \
+  hipLaunchKernelGGL((k_mx_route_xprep<XDT, CPW, ENT>), dim3(static_cast<unsigned>(k + 1), 2), dim3(64 * kMxRowWaves), \
+                     0, s, reinterpret_cast<const void *>(x), tab, reinterpret_cast<const void *>(logits), logits_dt,  \
+                     reinterpret_cast<const float *>(bias), static_cast<int>(E), k, scale, H, idx, wts, m.pos,         \
+                     m.row_map, m.tiles, m.ntiles, m.groups, m.ngroups, m.xp, m.xs)
+#define RX(XDT, CPW)                                       \
+  do {                                                     \
+    if (E <= 320) RXE(XDT, CPW, 5); else RXE(XDT, CPW, 16); \
+  } while (0)
+    VYBDQ_DISPATCH_IN(x_dt, XDT, {
+      if (cpw_h <= 1) RX(XDT, 1); else if (cpw_h <= 2) RX(XDT, 2); else if (cpw_h <= 4) RX(XDT, 4); else RX(XDT, 8);
+    });
+#undef RX
+#undef RXE
+    rc = check_launch("moe exl3 route and x rotation");
+    if (rc) return rc;
+  } else {
+    rc = moe_route_bucket(reinterpret_cast<const void *>(logits), logits_dt, reinterpret_cast<const float *>(bias), T, E,
+                          topk, scale, p.BP, idx, wts, m.pos, m.row_map, m.tiles, m.ntiles, m.groups, m.ngroups, s);
+    if (rc) return rc;
 #define XP(XDT, CPW)                                                                                            \
   hipLaunchKernelGGL((k_mx_xprep<XDT, CPW>), dim3(static_cast<unsigned>(n), 2), dim3(64 * kMxRowWaves), 0, s,      \
                      reinterpret_cast<const void *>(x), tab, idx, m.pos, k, H, n, m.xp, m.xs)
-  VYBDQ_DISPATCH_IN(x_dt, XDT, {
-    if (cpw_h <= 1) XP(XDT, 1); else if (cpw_h <= 2) XP(XDT, 2); else if (cpw_h <= 4) XP(XDT, 4); else XP(XDT, 8);
-  });
+    VYBDQ_DISPATCH_IN(x_dt, XDT, {
+      if (cpw_h <= 1) XP(XDT, 1); else if (cpw_h <= 2) XP(XDT, 2); else if (cpw_h <= 4) XP(XDT, 4); else XP(XDT, 8);
+    });
 #undef XP
-  rc = check_launch("moe exl3 x rotation");
-  if (rc) return rc;
+    rc = check_launch("moe exl3 x rotation");
+    if (rc) return rc;
+  }
   // 3. gate | up products
   MxGemmArgs ga{};
   ga.tab = tab;
