@@ -169,9 +169,11 @@ __device__ __forceinline__ void mx_load_row(const void *__restrict__ X, int64_t 
 // One token: its routing, its rows' groups and their rotations in one launch. Workgroup (slot, p) repeats
 // the routing for itself (route_wg_keys / route_wg_select: the same keys, selection and weights as the launch
 // of its own) with its x elements already in flight, and rotates that slot's row; workgroup (topk, 0) writes
-// the routing outputs and the groups. Both parts are latency: 6.3 us + 5.0 us and the gap between them as two launches, 9.1 us as one (288
-// experts, H = 4096: layer 69.0 -> 66.7 us, in a graph 60 -> 57.4; 1024 experts 37.3 -> 33.9; 64 slots 88.8 -> 81.8). Only
-// at one token: with more, a row's place depends on every token's routing.
+// the routing outputs and the groups. Both parts are latency: 6.3 us + 5.0 us and the gap between them as two
+// launches, 9.1 us as one (288 experts, H = 4096, I = 2048: layer 69.0 -> 66.7 us, its routed part in a graph
+// 59.7 -> 57.3; 512 experts, I = 1024 47.5 -> 47.4; 1024 experts, I = 512 36.6 -> 34.1; 64 of 320 experts,
+// H = 2048, I = 512 85.3 -> 81.4). Only at one token: with more, a row's place depends on every token's
+// routing.
 template <int XDT, int CPW, int ENT>
 __global__ void __launch_bounds__(64 * kMxRowWaves) k_mx_route_xprep(
     const void *__restrict__ X, const uint64_t *__restrict__ tab, const void *__restrict__ logits, int ldt,
