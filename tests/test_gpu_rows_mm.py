@@ -7,6 +7,7 @@ import torch
 
 from oracle import iquants, kquants, matmul
 from tests.test_gpu_gguf import gate, to_dev, x_as
+from tests.test_gpu_kquant import _x_pattern
 from vybforge_amd import ops, synth
 from vybforge_amd._lib import call, lib
 
@@ -110,3 +111,23 @@ def test_rows_gemm_falls_back(dev, ty):
          torch.cuda.current_stream().cuda_stream)
     assert matmul.rel_maxnorm(y.cpu().numpy(), ref) < matmul.TOL
     assert lib.vybdq_gemm_workspace_size(ty, M, N, K) == ws.nbytes
+
+
+@pytest.mark.parametrize("kind", ["fp16_limit", "tiny", "huge"])
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+@pytest.mark.parametrize("ty,N,K,at", [(ops.GGML_Q4_0, 208, 768, 0), (ops.GGML_Q8_0, 1040, 256, 0),
+                                       (ops.GGML_Q8_0, 64, 53248, 0), (ops.GGML_Q4_K, 128, 1024, 4),
+                                       (ops.GGML_Q5_K, 192, 512, 4), (ops.GGML_Q8_0, 256, 512, 4)])
+def test_gemm_64_rows_off_the_rows_path(dev, ty, N, K, at, xdt, kind):
+    """64 rows that k_rows_mm does not take (N % 64, no plan for the K, weights at a 4-byte address) keep the row
+    scales of X: activations of any magnitude neither overflow nor flush to zero."""
+    M = 64
+    rng = np.random.default_rng(ty + N + at + len(kind))
+    raw, w = weights(ty, rng, N, K)
+    xd, x64 = x_as(_x_pattern(kind, rng, M, K), xdt, dev)
+    W = torch.zeros(raw.size + 16, dtype=torch.uint8, device=dev)[at:at + raw.size]
+    W[:] = to_dev(raw, dev)
+    ws = ops.GemmWorkspace([(M, N, K)], dev, ty)
+    y = ops.gemm(ty, W, xd.reshape(M, K), N, K, workspace=ws).cpu().numpy()
+    assert np.all(np.isfinite(y))
+    assert matmul.rel_maxnorm(y, matmul.gemm_rows_f64(x64.reshape(M, K), w)) < matmul.TOL

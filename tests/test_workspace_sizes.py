@@ -1,0 +1,20 @@
+"""The workspace sizes that the library names cover every path a call of that size can take. CPU only."""
+
+import pytest
+
+from vybforge_amd import _lib
+
+ALL = [2, 8, 12, 13, 14, 22]
+
+
+def gemm_size(ty, M, N, K):
+    return _lib.lib.vybdq_gemm_workspace_size(ty, M, N, K)
+
+
+@pytest.mark.parametrize("ty", [2, 8, 12, 13])
+@pytest.mark.parametrize("N,K", [(1040, 5120), (5136, 17408), (1088, 5120), (5120, 28672), (64, 53248), (64, 256)])
+def test_gemm_64_rows_hold_the_scaled_copy_of_x(ty, N, K):
+    """From 64 rows the register bodies convert X into the workspace, row by row scaled; which body a call takes also
+    depends on what the query does not see (the alignment of W), so there is room for the copy at every shape."""
+    for M in (64, 65):
+        assert gemm_size(ty, M, N, K) >= M * K * 2 + M * 4

@@ -23,6 +23,7 @@
 // matrix, and y = silu(min(g, L)) * clamp(u, -L, L) (native/glm53/moe_ref.py:81-84).
 #include "gemv_dev.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace vybdq {
@@ -458,18 +459,20 @@ static int gemm_check(int wtype, uint64_t W, uint64_t X, uint64_t Y, int64_t M, 
   return VYBDQ_OK;
 }
 
-// what the fused bodies use (0: nothing)
+// what the fused bodies use (0: nothing). At 64 rows a call that rows_mm.h does not take (N % 64, W not 16-byte
+// aligned, a K that fits no plan) runs on the register bodies, which scale X only into a workspace that holds its copy.
 static int64_t fused_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
-  if (M >= 1 && M <= kRowsMmMax && N >= 64 && K >= 256) return rows_mm_workspace_size(wtype, M, N, K);
   if (wtype == 14 || wtype == 22) return M >= 1 && N >= 64 && K >= 256 ? kq2_workspace_size(wtype, M, N, K) : 0;
   if ((wtype != 2 && wtype != 8 && wtype != 12 && wtype != 13) || M < 64 || !mmq_supported(M, N, K)) return 0;
   return mmq_workspace_size(wtype, M, N, K);
 }
 
 extern "C" int64_t vybdq_gemm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
+  const bool ok = M >= 1 && N >= 64 && K >= 256;
   const int64_t fused = fused_workspace_size(wtype, M, N, K);
-  const int64_t wide = M >= 1 && N >= 64 && K >= 256 ? wide_mm_workspace_size(wtype, M, N, K) : 0;
-  return wide > fused ? wide : fused;
+  const int64_t rows = ok && M <= kRowsMmMax ? rows_mm_workspace_size(wtype, M, N, K) : 0;
+  const int64_t wide = ok && M > kRowsMmMax ? wide_mm_workspace_size(wtype, M, N, K) : 0;
+  return std::max({fused, rows, wide});
 }
 
 extern "C" int vybdq_gemm_ws(int wtype, uint64_t W, uint64_t X, uint64_t Y, int64_t M, int64_t N, int64_t K,
