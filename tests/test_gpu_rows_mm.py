@@ -95,7 +95,8 @@ def test_rows_gemm_ranges(dev, ty, xdt):
 
 @pytest.mark.parametrize("ty", [ops.GGML_Q4_K, ops.GGML_Q6_K])
 def test_rows_gemm_falls_back(dev, ty):
-    """Weights at a 4-byte address and a workspace that is too small take the general tiles."""
+    """Weights at a 4-byte address take the general tiles; a workspace too small for the planned partials takes a plan
+    with fewer K ranges."""
     M, N, K = 24, 256, 1024
     rng = np.random.default_rng(ty)
     raw, w = weights(ty, rng, N, K)
@@ -111,6 +112,27 @@ def test_rows_gemm_falls_back(dev, ty):
          torch.cuda.current_stream().cuda_stream)
     assert matmul.rel_maxnorm(y.cpu().numpy(), ref) < matmul.TOL
     assert lib.vybdq_gemm_workspace_size(ty, M, N, K) == ws.nbytes
+
+
+@pytest.mark.parametrize("ty", TYPES)
+@pytest.mark.parametrize("N,K,Mmax", [(256, 4352, 64), (320, 1280, 33), (128, 2560, 300)])
+def test_rows_gemm_one_workspace(dev, ty, N, K, Mmax):
+    """One workspace sized for the largest row count serves the smaller ones on k_rows_mm, and so does half of it
+    (fewer K ranges): bf16 activations past fp16's range, which the general tiles would convert as they are, match."""
+    rng = np.random.default_rng(ty + N + Mmax)
+    raw, w = weights(ty, rng, N, K)
+    xd, x64 = x_as((rng.standard_normal((Mmax, K)) * 1e6).astype(np.float32), "bf16", dev)
+    Wd, x64 = to_dev(raw, dev), x64.reshape(Mmax, K)
+    ws = ops.GemmWorkspace([(Mmax, N, K)], dev, ty)
+    ref = matmul.gemm_rows_f64(x64, w)
+    for M in (1, 9, 16, 17, 24, 31, 32, 33, 48, 63, 64):
+        if M > Mmax:
+            continue
+        for part in (1, 2):
+            y = torch.zeros((M, N), dtype=torch.float32, device=dev)
+            call("vybdq_gemm_ws", ty, Wd.data_ptr(), xd.data_ptr(), y.data_ptr(), M, N, K, ops.BF16, ops.F32, 0, 0,
+                 ws.ptr, ws.nbytes // part, torch.cuda.current_stream().cuda_stream)
+            assert matmul.rel_maxnorm(y.cpu().numpy(), ref[:M]) < matmul.TOL, (M, part)
 
 
 @pytest.mark.parametrize("kind", ["fp16_limit", "tiny", "huge"])

@@ -18,3 +18,15 @@ def test_gemm_64_rows_hold_the_scaled_copy_of_x(ty, N, K):
     depends on what the query does not see (the alignment of W), so there is room for the copy at every shape."""
     for M in (64, 65):
         assert gemm_size(ty, M, N, K) >= M * K * 2 + M * 4
+
+
+@pytest.mark.parametrize("ty", ALL)
+@pytest.mark.parametrize("N,K", [(2560, 9728), (5120, 17408), (17408, 5120), (1024, 5120), (320, 768), (64, 256),
+                                 (4096, 53248), (9728, 2560)])
+def test_gemm_few_rows_size_covers_smaller_batches(ty, N, K):
+    """One workspace for the largest batch serves every smaller one: up to 64 rows the size never falls as rows are
+    added, and a longer call's holds that of 64 rows."""
+    sizes = [gemm_size(ty, M, N, K) for M in range(1, 65)]
+    assert sizes[0] > 0 or N * K > 1 << 26
+    assert sizes == sorted(sizes)
+    assert all(gemm_size(ty, M, N, K) >= sizes[62] for M in (64, 65, 96, 200, 512))

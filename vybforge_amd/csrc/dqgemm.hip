@@ -470,7 +470,7 @@ static int64_t fused_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) 
 extern "C" int64_t vybdq_gemm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
   const bool ok = M >= 1 && N >= 64 && K >= 256;
   const int64_t fused = fused_workspace_size(wtype, M, N, K);
-  const int64_t rows = ok && M <= kRowsMmMax ? rows_mm_workspace_size(wtype, M, N, K) : 0;
+  const int64_t rows = ok ? rows_mm_workspace_size(wtype, std::min(M, kRowsMmMax), N, K) : 0;
   const int64_t wide = ok && M > kRowsMmMax ? wide_mm_workspace_size(wtype, M, N, K) : 0;
   return std::max({fused, rows, wide});
 }

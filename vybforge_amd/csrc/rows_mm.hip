@@ -1,6 +1,8 @@
 // Host side of the GEMM at a few X rows (rows_mm.h): plan, dispatch and the split reduce.
 #include "rows_mm.h"
 
+#include <algorithm>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 
@@ -38,10 +40,10 @@ struct RowsPlan {
 // need the registers of 8 waves; and so may LDS (Q8_0: two stages of 256 rows and one X super-block are all
 // of it). One workgroup fits a CU; the plan minimises the stages of the busiest CU (a stage's bytes at
 // the 18.5 GB/s a CU gets of HBM) plus a workgroup's start (X staging) and the split partials, written
-// and read back. With only two LDS stages a stage is barely in flight: 10% more. VYBDQ_ROWS_PLAN="sps,nwg"
-// overrides the split (ignored where it does not fit).
+// and read back. With only two LDS stages a stage is barely in flight: 10% more. Only plans whose partials
+// fit ws_bytes are looked at. VYBDQ_ROWS_PLAN="sps,nwg" overrides the split (ignored where it does not fit).
 template <int FMT>
-static RowsPlan rows_plan(int M, int64_t N, int64_t K, bool split) {
+static RowsPlan rows_plan(int M, int64_t N, int64_t K, int64_t ws_bytes) {
   using F = RowsFmt<FMT>;
   const int SB = static_cast<int>(K / 256), MF = (M + 15) / 16, cus = 256;
   const int xsb = MF * (F::OPS * 1024 + 64), tab = FMT == FMT_IQ2_S ? kRowsGrid : 0;
@@ -58,7 +60,7 @@ static RowsPlan rows_plan(int M, int64_t N, int64_t K, bool split) {
       int ns = (160 * 1024 - tab - sps * xsb) / stage;
       if (ns < 2) break;
       ns = ns > 4 ? 4 : ns;
-      if (splits > (split ? kRowsMaxSplits : 1)) continue;
+      if (splits > kRowsMaxSplits || (splits > 1 && splits * M * N * 4 > ws_bytes)) continue;
       int nwg = cus / splits > 0 ? cus / splits : 1;
       if (fs) {
         if (sps != (fs < SB ? fs : SB)) continue;
@@ -84,23 +86,29 @@ bool rows_mm_supported(int wtype, int64_t M, int64_t N, int64_t K) {
 }
 
 // the plan of a type id
-static RowsPlan rows_plan_ty(int wtype, int M, int64_t N, int64_t K, bool split) {
+static RowsPlan rows_plan_ty(int wtype, int M, int64_t N, int64_t K, int64_t ws_bytes) {
   switch (wtype) {
-    case 2: return rows_plan<FMT_Q4_0>(M, N, K, split);
-    case 8: return rows_plan<FMT_Q8_0>(M, N, K, split);
-    case 12: return rows_plan<FMT_Q4_K>(M, N, K, split);
-    case 13: return rows_plan<FMT_Q5_K>(M, N, K, split);
-    case 14: return rows_plan<FMT_Q6_K>(M, N, K, split);
-    default: return rows_plan<FMT_IQ2_S>(M, N, K, split);
+    case 2: return rows_plan<FMT_Q4_0>(M, N, K, ws_bytes);
+    case 8: return rows_plan<FMT_Q8_0>(M, N, K, ws_bytes);
+    case 12: return rows_plan<FMT_Q4_K>(M, N, K, ws_bytes);
+    case 13: return rows_plan<FMT_Q5_K>(M, N, K, ws_bytes);
+    case 14: return rows_plan<FMT_Q6_K>(M, N, K, ws_bytes);
+    default: return rows_plan<FMT_IQ2_S>(M, N, K, ws_bytes);
   }
 }
 
-// workspace: split partials (at least 256 bytes where the shape is taken, so that a caller has one)
+// Workspace: the split partials of M rows and of every smaller count, so that one workspace serves a batch that shrinks
+// (at least 256 bytes where the shape is taken, so that a caller has one). Within 16 row counts a plan's estimate is
+// a constant plus a term in splits times rows, so its splits only fall as rows are added: those of the first count bound
+// the rest.
 int64_t rows_mm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
   if (!rows_mm_supported(wtype, M, N, K)) return 0;
-  const RowsPlan p = rows_plan_ty(wtype, static_cast<int>(M), N, K, true);
-  if (p.splits == 0) return 0;
-  return p.splits > 1 ? static_cast<int64_t>(p.splits) * M * N * 4 : 256;
+  int64_t need = 0;
+  for (int64_t m = 1; m <= M; m += 16) {
+    const int64_t splits = rows_plan_ty(wtype, static_cast<int>(m), N, K, INT64_MAX).splits, last = m + 15 < M ? m + 15 : M;
+    if (splits > 0) need = std::max(need, splits > 1 ? splits * last * N * 4 : 256);
+  }
+  return need;
 }
 
 template <int FMT, int XDT, int MF, int NW>
@@ -138,8 +146,8 @@ static int rows_launch_x(const RowsArgs &a, const RowsPlan &p, hipStream_t s) {
 template <int FMT>
 static int rows_run_fmt(RowsArgs &a, int xdt, void *ws, int64_t ws_bytes, hipStream_t s) {
   const int64_t K = static_cast<int64_t>(a.SB) * 256;
-  const RowsPlan p = rows_plan<FMT>(a.M, a.N, K, ws != nullptr);
-  if (p.splits == 0 || (p.splits > 1 && ws_bytes < static_cast<int64_t>(p.splits) * a.M * a.N * 4)) return 1;
+  const RowsPlan p = rows_plan<FMT>(a.M, a.N, K, ws_bytes);
+  if (p.splits == 0) return 1;
   a.rowbytes = unit_row_bytes<FMT>(K / 64);
   a.splits = p.splits;
   a.sps = p.sps;
