@@ -49,19 +49,21 @@ def test_rows_gemm(dev, ty, M, N, K):
 
 
 @pytest.mark.parametrize("ty", TYPES)
-@pytest.mark.parametrize("plan", ["1,1", "2,3", "3,2", "9,1"])
-def test_rows_gemm_plans(dev, monkeypatch, ty, plan):
+@pytest.mark.parametrize("plan,K,splits", [("1,1", 1792, 7), ("2,3", 1792, 4), ("3,2", 1792, 3), ("9,1", 1024, 1)])
+def test_rows_gemm_plans(dev, monkeypatch, ty, plan, K, splits):
     """Forced K ranges and workgroups per range: several tiles per workgroup (the LDS stages run on across
-    tiles), a ragged last range, one range; f64 output with a residual and a wider row stride."""
+    tiles), a ragged last range, one range (a K whose X fits LDS for every type); f64 output with a residual and a
+    wider row stride."""
     monkeypatch.setenv("VYBDQ_TUNING", "1")
     monkeypatch.setenv("VYBDQ_ROWS_PLAN", plan)
-    M, N, K, ldy = 21, 896, 1792, 1000
+    M, N, ldy = 21, 896, 1000
     rng = np.random.default_rng(ty + len(plan))
     raw, w = weights(ty, rng, N, K)
     x = synth.activations(rng, (M, K)).astype(np.float16)
     rs = synth.activations(rng, (M, ldy)).astype(np.float64)
     Wd, Xd, y = to_dev(raw, dev), to_dev(x, dev), to_dev(rs, dev)
     ws = ops.GemmWorkspace([(M, N, K)], dev, ty)
+    assert ws.nbytes == (splits * M * N * 4 if splits > 1 else 256)  # the forced plan
     call("vybdq_gemm_ws", ty, Wd.data_ptr(), Xd.data_ptr(), y.data_ptr(), M, N, K, ops.F16, ops._dt(torch.float64), ldy,
          y.data_ptr(), ws.ptr, ws.nbytes, torch.cuda.current_stream().cuda_stream)
     got = y.cpu().numpy()

@@ -30,3 +30,14 @@ def test_gemm_few_rows_size_covers_smaller_batches(ty, N, K):
     assert sizes[0] > 0 or N * K > 1 << 26
     assert sizes == sorted(sizes)
     assert all(gemm_size(ty, M, N, K) >= sizes[62] for M in (64, 65, 96, 200, 512))
+
+
+@pytest.mark.parametrize("ty", ALL)
+@pytest.mark.parametrize("plan", ["9,1", "40,1", "99,3", "0,1", "x"])
+def test_gemm_few_rows_override_that_does_not_fit(monkeypatch, ty, plan):
+    """A tuning override whose K range does not fit LDS (or that is none) leaves the planner's choice."""
+    own = gemm_size(ty, 64, 512, 53248)
+    own21 = gemm_size(ty, 21, 896, 12800)
+    monkeypatch.setenv("VYBDQ_ROWS_PLAN", plan)
+    assert gemm_size(ty, 64, 512, 53248) == own
+    assert gemm_size(ty, 21, 896, 12800) == own21 > 0

@@ -52,32 +52,32 @@ static RowsPlan rows_plan(int M, int64_t N, int64_t K, int64_t ws_bytes) {
   int fs = 0, fn = 0;
   if (const char *e = tuning_env("VYBDQ_ROWS_PLAN"))
     if (sscanf(e, "%d,%d", &fs, &fn) != 2 || fs < 1 || fn < 1) fs = fn = 0;
-  for (int NW = MF <= 2 ? 16 : 8; NW >= 4; NW /= 2) {
-    const int BN = 16 * NW, tiles = static_cast<int>(N / BN), stage = BN * F::C * 16;
-    if (N % BN || (NW == 4 && N % 128 == 0)) continue;  // 4 waves only where 8 do not divide N
-    for (int sps = 1; sps <= SB && sps <= 32; ++sps) {
-      const int splits = (SB + sps - 1) / sps;
-      int ns = (160 * 1024 - tab - sps * xsb) / stage;
-      if (ns < 2) break;
-      ns = ns > 4 ? 4 : ns;
-      if (splits > kRowsMaxSplits || (splits > 1 && splits * M * N * 4 > ws_bytes)) continue;
-      int nwg = cus / splits > 0 ? cus / splits : 1;
-      if (fs) {
-        if (sps != (fs < SB ? fs : SB)) continue;
-        nwg = fn;
-      }
-      nwg = nwg < tiles ? nwg : tiles;
-      const int rounds = (splits * nwg + cus - 1) / cus, stages = (tiles + nwg - 1) / nwg * sps;
-      double t = rounds * (stages * stage / 18.5e3 * (ns == 2 ? 1.1 : 1.0) + 2.5 + 0.2 * sps * MF);
-      if (NW < 16 && MF <= 2) t *= 1.08;
-      if (splits > 1) t += 4.0 + 8.0 * splits * M * static_cast<double>(N) / 4.0e6;
-      if (best_t < 0 || t < best_t) {
-        best_t = t;
-        best = {NW, splits, sps, nwg, ns};
+  if (fs > SB) fs = SB;
+  for (;; fs = 0) {
+    for (int NW = MF <= 2 ? 16 : 8; NW >= 4; NW /= 2) {
+      const int BN = 16 * NW, tiles = static_cast<int>(N / BN), stage = BN * F::C * 16;
+      if (N % BN || (NW == 4 && N % 128 == 0)) continue;  // 4 waves only where 8 do not divide N
+      for (int sps = fs ? fs : 1; sps <= SB && sps <= (fs ? fs : 32); ++sps) {
+        const int splits = (SB + sps - 1) / sps;
+        int ns = (160 * 1024 - tab - sps * xsb) / stage;
+        if (ns < 2) break;
+        ns = ns > 4 ? 4 : ns;
+        if (splits > kRowsMaxSplits || (splits > 1 && splits * M * N * 4 > ws_bytes)) continue;
+        int nwg = cus / splits > 0 ? cus / splits : 1;
+        if (fs) nwg = fn;
+        nwg = nwg < tiles ? nwg : tiles;
+        const int rounds = (splits * nwg + cus - 1) / cus, stages = (tiles + nwg - 1) / nwg * sps;
+        double t = rounds * (stages * stage / 18.5e3 * (ns == 2 ? 1.1 : 1.0) + 2.5 + 0.2 * sps * MF);
+        if (NW < 16 && MF <= 2) t *= 1.08;
+        if (splits > 1) t += 4.0 + 8.0 * splits * M * static_cast<double>(N) / 4.0e6;
+        if (best_t < 0 || t < best_t) {
+          best_t = t;
+          best = {NW, splits, sps, nwg, ns};
+        }
       }
     }
+    if (!fs || best.splits) return best;  // splits = 0: no plan fits (an override that does not fit: plan without it)
   }
-  return best;  // splits = 0: no plan fits
 }
 
 bool rows_mm_supported(int wtype, int64_t M, int64_t N, int64_t K) {
@@ -154,14 +154,9 @@ static int rows_run_fmt(RowsArgs &a, int xdt, void *ws, int64_t ws_bytes, hipStr
   a.ns = p.ns;
   a.tiles = a.N / (16 * p.NW);
   a.part = static_cast<float *>(ws);
-#ifdef ROWS_PROBE
-  if (xdt != VYBDQ_BF16) return 1;
-  return rows_launch_x<FMT, VYBDQ_BF16>(a, p, s);
-#else
   int rc = VYBDQ_OK;
   VYBDQ_DISPATCH_IN(xdt, XDT, rc = rows_launch_x<FMT, XDT>(a, p, s));
   return rc;
-#endif
 }
 
 // Returns 1 when the call does not fit (shape, W not 16-byte aligned).
