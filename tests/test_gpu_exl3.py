@@ -130,6 +130,25 @@ def test_exl3_gemm_step_remainders(dev, K, N, B):
     assert matmul.rel_maxnorm(y, ref) < matmul.TOL
 
 
+def test_exl3_gemm_workspace_of_a_larger_batch(dev):
+    """A workspace of the size named for 4 rows takes every smaller batch (their K splits may be more)."""
+    K, N = 1152, 7296
+    rng = np.random.default_rng(9)
+    t, suh, svh = synth.exl3_tensors(rng, K, N)
+    td, sud, svd = dev_t(t, dev), dev_t(suh, dev), dev_t(svh, dev)
+    nbytes = _lib.lib.vybdq_exl3_workspace_size(4, K, N)
+    ws = torch.zeros(nbytes + 256, dtype=torch.uint8, device=dev)
+    wp = (ws.data_ptr() + 255) // 256 * 256
+    x = rng.standard_normal((4, K)).astype(np.float16)
+    xd = dev_t(x, dev)
+    ref = x.astype(np.float64) @ exl3.dequant_exl3_f64(t, suh, svh)
+    for B in (4, 2, 1, 3):
+        y = torch.empty((B, N), dtype=torch.float32, device=dev)
+        _lib.call("vybdq_exl3_gemm", td.data_ptr(), sud.data_ptr(), svd.data_ptr(), xd.data_ptr(), y.data_ptr(), B, K, N,
+                  _lib.EXL3_MCG, ops.F16, ops.F32, wp, nbytes, torch.cuda.current_stream().cuda_stream)
+        assert matmul.rel_maxnorm(y.cpu().numpy(), ref[:B]) < matmul.TOL
+
+
 def test_exl3_gemm_graph_replays(dev):
     """Captured once, replayed with other work between the replays: every replay matches eager."""
     rng = np.random.default_rng(7)

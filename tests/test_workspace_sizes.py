@@ -41,3 +41,12 @@ def test_gemm_few_rows_override_that_does_not_fit(monkeypatch, ty, plan):
     monkeypatch.setenv("VYBDQ_ROWS_PLAN", plan)
     assert gemm_size(ty, 64, 512, 53248) == own
     assert gemm_size(ty, 21, 896, 12800) == own21 > 0
+
+
+def test_exl3_size_covers_smaller_batches():
+    """vybdq_exl3_gemm refuses a workspace below its need: the size for a batch holds every smaller one's."""
+    f = _lib.lib.vybdq_exl3_workspace_size
+    for K in (128, 256, 384, 1152, 1920, 2048, 4096, 5120, 17408):
+        for N in (128, 256, 768, 1024, 5120, 14848, 17408, 26624, 131072):
+            sizes = [f(B, K, N) for B in range(1, 17)]
+            assert sizes == sorted(sizes), (K, N)

@@ -20,6 +20,7 @@
 // N (one 128-column Hadamard block) and reads 1 KB of contiguous trellis per step.
 #include "exl3_dev.h"
 
+#include <algorithm>
 #include <cstdlib>
 
 namespace vybdq {
@@ -430,9 +431,12 @@ extern "C" int vybdq_dequant_exl3(uint64_t trellis, uint64_t suh, uint64_t svh, 
   return check_launch("vybdq_dequant_exl3");
 }
 
+// also what every smaller batch needs (its K splits may be more), so that one workspace serves them all
 extern "C" int64_t vybdq_exl3_workspace_size(int64_t B, int64_t K, int64_t N) {
   if (B < 1 || B > 16 || K <= 0 || N <= 0 || K % 128 || N % 128) return -1;
-  return exl3_ws_bytes(B, K, N);
+  int64_t need = exl3_ws_bytes(B, K, N);
+  for (int64_t b = 1; b < B; b *= 2) need = std::max(need, exl3_ws_bytes(b, K, N));
+  return need;
 }
 
 template <bool FUSED>
