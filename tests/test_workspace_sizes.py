@@ -50,3 +50,14 @@ def test_exl3_size_covers_smaller_batches():
         for N in (128, 256, 768, 1024, 5120, 14848, 17408, 26624, 131072):
             sizes = [f(B, K, N) for B in range(1, 17)]
             assert sizes == sorted(sizes), (K, N)
+
+
+def test_moe_exl3_size_covers_fewer_tokens():
+    """vybdq_moe_forward_exl3 refuses a workspace below its need: the size for T tokens holds that of fewer."""
+    f = _lib.lib.vybdq_moe_exl3_workspace_size
+    Ts = list(range(1, 34)) + [48, 63, 64, 65, 100, 128, 200, 256, 512, 1024]
+    for H, I in ((256, 256), (256, 1536), (512, 2048), (1024, 512), (2560, 1024), (4096, 2048)):
+        for E in (8, 12, 96, 288):
+            for k in (1, 4, 8):
+                sizes = [f(T, H, I, E, k) for T in Ts]
+                assert sizes == sorted(sizes), (H, I, E, k)

@@ -39,6 +39,8 @@
 #include "exl3_dev.h"
 #include "moe_route.h"
 
+#include <algorithm>
+
 namespace vybdq {
 
 // moe.hip
@@ -747,7 +749,15 @@ static bool mx_shape_ok(int64_t T, int64_t H, int64_t I, int64_t E, int64_t topk
 
 extern "C" int64_t vybdq_moe_exl3_workspace_size(int64_t T, int64_t H, int64_t I, int64_t E, int64_t topk) {
   if (!mx_shape_ok(T, H, I, E, topk)) return -1;
-  return mx_layout(nullptr, mx_plan(T, H, I, E, topk), T, H, I, topk).bytes;
+  // also what every smaller token count needs, so that one workspace serves them all: the splits only fall as
+  // tokens are added, and once all are one the layout only grows
+  int64_t need = mx_layout(nullptr, mx_plan(T, H, I, E, topk), T, H, I, topk).bytes;
+  for (int64_t t = 1; t < T; ++t) {
+    const MxPlan p = mx_plan(t, H, I, E, topk);
+    need = std::max(need, mx_layout(nullptr, p, t, H, I, topk).bytes);
+    if (p.gu.S == 1 && p.dn.S == 1 && p.Ssg == 1 && p.Ssd == 1) break;
+  }
+  return need;
 }
 
 extern "C" int vybdq_moe_forward_exl3(uint64_t x, int x_dt, uint64_t logits, int logits_dt, uint64_t bias,

@@ -545,15 +545,15 @@ class MoeExl3Layer:
         _need(bias is None or (bias.numel() == E and bias.dtype == torch.float32), "bias must be float32 [E]")
         self.H, self.I, self.E, self.topk = H, I, E, topk
         self.shared, self.scale, self.limit, self.bias = shared, scale, limit, bias
-        self._ws, self._ws_bytes = None, 0
+        self._ws, self._ws_bytes, self._ws_t = None, 0, 0
 
     def _workspace(self, T, device):
-        n = _lib.lib.vybdq_moe_exl3_workspace_size(T, self.H, self.I, self.E, self.topk)
-        if n < 0:
-            raise ValueError("unsupported MoE shape")
-        if self._ws is None or self._ws_bytes < n:
+        if not 0 < T <= self._ws_t:  # the size for T tokens covers fewer
+            n = _lib.lib.vybdq_moe_exl3_workspace_size(T, self.H, self.I, self.E, self.topk)
+            if n < 0:
+                raise ValueError("unsupported MoE shape")
             self._ws = torch.empty(n + 256, dtype=torch.uint8, device=device)
-            self._ws_bytes = n
+            self._ws_bytes, self._ws_t = n, T
         return (self._ws.data_ptr() + 255) // 256 * 256, self._ws_bytes
 
     def __call__(self, x, logits, out_dtype=torch.float32, out=None, routing=False):
