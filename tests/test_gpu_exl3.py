@@ -149,6 +149,20 @@ def test_exl3_gemm_workspace_of_a_larger_batch(dev):
         assert matmul.rel_maxnorm(y.cpu().numpy(), ref[:B]) < matmul.TOL
 
 
+@pytest.mark.parametrize("K,B,splits", [(17408, 2, "1"), (39936, 2, "1"), (65536, 2, "1")])
+def test_exl3_gemm_long_splits(dev, monkeypatch, K, B, splits):
+    """A split whose x' rows pass 64 KB of LDS (70 KB, 160 KB), as matrices of few splits and many columns have
+    them, and a forced one that would pass the CU's 160 KB (not taken)."""
+    monkeypatch.setenv("VYBDQ_EXL3_SPLITS", splits)
+    N = 128
+    rng = np.random.default_rng(K)
+    t, suh, svh = synth.exl3_tensors(rng, K, N)
+    lin = ops.Exl3Linear(dev_t(t, dev), dev_t(suh, dev), dev_t(svh, dev), K, N, max_batch=B)
+    x = rng.standard_normal((B, K)).astype(np.float16)
+    y = lin(dev_t(x, dev)).cpu().numpy()
+    assert matmul.rel_maxnorm(y, x.astype(np.float64) @ exl3.dequant_exl3_f64(t, suh, svh)) < matmul.TOL
+
+
 def test_exl3_gemm_graph_replays(dev):
     """Captured once, replayed with other work between the replays: every replay matches eager."""
     rng = np.random.default_rng(7)

@@ -32,6 +32,7 @@ __host__ __device__ constexpr bool exl3_fused(int BP) { return BP <= 2; }
 // LDS of the fused GEMM: batch <= 2 the x' stage of a split (fp16, rows exl3_xstride apart), reused
 // after the loop for the waves' partials [4][batch rows][kExl3RedStride]; larger batches those alone
 __host__ __device__ constexpr int exl3_xstride(int kbs) { return 16 * kbs + 8; }
+constexpr size_t kExl3MaxLds = 160 * 1024 - 256;  // dynamic, beside the kernel's static words
 static size_t exl3_lds_bytes(int BP, int kbs) {
   const size_t main = exl3_fused(BP) ? static_cast<size_t>(BP) * exl3_xstride(kbs) * 2 : 0;
   const size_t red = static_cast<size_t>(4) * BP * kExl3RedStride * 4;
@@ -340,11 +341,15 @@ static Exl3Split exl3_splits(int64_t K, int64_t N, int BP) {
   int64_t best_cost = -1;
   for (int S = 1; S <= 16; ++S) {
     const Exl3Split c = shape(S);
+    if (exl3_lds_bytes(BP, c.kbs) > kExl3MaxLds) continue;
     const int64_t rounds = (groups * c.S + 255) / 256;
     const int64_t cost = exl3_fused(BP) ? rounds * (8 * c.kbs + 16) + BP * c.kbs : rounds * (8 * c.kbs + 48) + 8 * c.S;
     if (best_cost < 0 || cost < best_cost) best_cost = cost, best = c;
   }
-  if (const char *e = tuning_env("VYBDQ_EXL3_SPLITS")) best = shape(atoi(e) > 0 ? atoi(e) : 1);  // tuning override
+  if (const char *e = tuning_env("VYBDQ_EXL3_SPLITS")) {  // tuning override
+    const Exl3Split c = shape(atoi(e) > 0 ? atoi(e) : 1);
+    if (exl3_lds_bytes(BP, c.kbs) <= kExl3MaxLds) best = c;
+  }
   return best;
 }
 
@@ -443,10 +448,10 @@ template <bool FUSED>
 static void exl3_gemm_launch(const uint16_t *t, const void *X, int xdt, const _Float16 *su, const _Float16 *sv,
                              void *Y, int ydt, int B, int BP, const _Float16 *xp, float *zp, uint32_t *arr, int64_t K,
                              int NB, const Exl3Split &sp, hipStream_t s) {
-  const size_t lds = exl3_lds_bytes(BP, sp.kbs);  // at most 82 KB (exl3_size_ok)
+  const size_t lds = exl3_lds_bytes(BP, sp.kbs);  // at most kExl3MaxLds (exl3_splits; exl3_size_ok: some split fits)
   if (lds > 64 * 1024) {
     static std::atomic<uint64_t> raised{0};
-    if (ensure_lds_limit(reinterpret_cast<const void *>(&k_exl3_gemm<FUSED>), 160 * 1024, raised, "exl3 gemm"))
+    if (ensure_lds_limit(reinterpret_cast<const void *>(&k_exl3_gemm<FUSED>), kExl3MaxLds, raised, "exl3 gemm"))
       return;  // the launch below then fails and check_launch reports it
   }
   hipLaunchKernelGGL((k_exl3_gemm<FUSED>), dim3(static_cast<unsigned>(NB / 8), static_cast<unsigned>(sp.S)),
