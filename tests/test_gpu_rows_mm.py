@@ -155,3 +155,34 @@ def test_gemm_64_rows_off_the_rows_path(dev, ty, N, K, at, xdt, kind):
     y = ops.gemm(ty, W, xd.reshape(M, K), N, K, workspace=ws).cpu().numpy()
     assert np.all(np.isfinite(y))
     assert matmul.rel_maxnorm(y, matmul.gemm_rows_f64(x64.reshape(M, K), w)) < matmul.TOL
+
+
+@pytest.mark.parametrize("ty", TYPES)
+@pytest.mark.parametrize("xdt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("M,N,K", [(11, 64, 512), (30, 256, 1792), (64, 128, 1280)])
+def test_rows_gemm_non_finite(dev, ty, xdt, M, N, K):
+    """Infinities and NaNs of X: one, several of one sign and of both, in one super-block and in two, beside a NaN.
+    Every output is what the sum over k gives (the infinity's sign, or NaN), and the other rows stay as they are."""
+    rng = np.random.default_rng(ty + M + len(xdt))
+    raw, w = weights(ty, rng, N, K)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[0, 5] = np.inf
+    x[1, 300] = -np.inf
+    x[2, [64, 70, 200]] = np.inf
+    x[4, [31, 32]] = np.inf, -np.inf
+    x[5, [100, K - 1]] = np.inf
+    x[6, [8, 264]] = -np.inf, np.inf
+    x[7, 17] = np.nan
+    x[8, [40, 41]] = np.inf, np.nan
+    x[M - 1, K - 256] = np.inf
+    xd, x64 = x_as(x, xdt, dev)
+    ws = ops.GemmWorkspace([(M, N, K)], dev, ty)
+    y = ops.gemm(ty, to_dev(raw, dev), xd.reshape(M, K), N, K, workspace=ws).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        terms = x64.reshape(M, 1, K) * np.asarray(w, dtype=np.float64)[None]
+        ref = terms.sum(-1)
+    bad = [0, 1, 2, 4, 5, 6, 7, 8, M - 1]
+    np.testing.assert_array_equal(y[bad], ref[bad].astype(np.float32))
+    assert not np.isfinite(y[bad]).any()
+    good = [m for m in range(M) if m not in bad]
+    assert matmul.rel_maxnorm(y[good], ref[good]) < matmul.TOL

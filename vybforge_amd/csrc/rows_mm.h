@@ -23,8 +23,10 @@
 // Measured with the reduce launch, 24 rows bf16, 17408 x 5120 and 5120 x 17408: Q4_K 25.3 and 26.2 us (65 and 136 on the
 // 64-row tiles of kqgemm.hip), Q6_K 32.6 and 34.1 (72 and 177), q4_0 23.3 and 24.1 (47 and 86). The loop
 // itself streams weights at 4.6 TB/s; the rest is the start (X), the last round of tiles and the
-// reduce (~5 us). Non-finite activations give non-finite outputs in their row (an infinity may come out as NaN: the
-// mins are subtracted apart from the products).
+// reduce (~5 us). Non-finite activations give what the sum over k gives: where the mins are subtracted apart from the
+// products (Q4_K, Q5_K), an infinity would meet zeros and infinities that the weight itself is not, so a row's
+// super-block that holds one is staged as zeros, marked by a negative scale, and its infinities (and NaNs) times their
+// whole weights are added on a path of their own.
 #pragma once
 #include "gemv_dev.h"
 
@@ -222,8 +224,9 @@ __global__ void __launch_bounds__(64 * NW) k_rows_mm(const RowsArgs a) {
     amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
     float inv;
     const float sc = block_scale(amax, inv);
+    const bool inf = F::MINS && amax == __builtin_inff();
     char *base = xs + (q / MF) * Sh::XSB + (q % MF) * (F::OPS * 1024);
-    if (g == 0) reinterpret_cast<float *>(xs + (q / MF) * Sh::XSB + MF * F::OPS * 1024)[16 * (q % MF) + n] = sc;
+    if (g == 0) reinterpret_cast<float *>(xs + (q / MF) * Sh::XSB + MF * F::OPS * 1024)[16 * (q % MF) + n] = inf ? -1.0f : sc;
 #pragma unroll
     for (int cc = 0; cc < 8; ++cc) {  // block cc of the super-block; this lane's chunk: quarter g
       u4 o;
@@ -263,6 +266,13 @@ __global__ void __launch_bounds__(64 * NW) k_rows_mm(const RowsArgs a) {
             p[4] = static_cast<_Float16>(0.f);
           }
         }
+      }
+    }
+    if constexpr (F::MINS) {
+      asm volatile("" ::: "memory");  // stored after the values above
+      if (inf) {  // this lane's operands and sums again, as zeros
+        for (int j = 0; j < 8; ++j) *reinterpret_cast<u4 *>(base + (4 * (j & 1) + g) * 1024 + (n + 16 * (j >> 1)) * 16) = u4{0u, 0u, 0u, 0u};
+        *reinterpret_cast<u4 *>(base + 8 * 1024 + (n + 16 * g) * 16) = u4{0u, 0u, 0u, 0u};
       }
     }
   };
@@ -350,9 +360,18 @@ __global__ void __launch_bounds__(64 * NW) k_rows_mm(const RowsArgs a) {
   for (int m = 0; m < MF; ++m) acc[m] = f4{0.f, 0.f, 0.f, 0.f};
   const int row0 = wave * 16 + n;  // this lane's weight row within the tile
   int tile = blockIdx.x, sbl = 0, cb = 0;
+  bool has_inf = false;  // a marked super-block among the workgroup's
   for (int z = 0; z < total; ++z) {
     wait_later(min(NS - 2, total - 1 - z));
     bar();
+    if constexpr (F::MINS) {
+      if (z == 0) {
+        bool neg = false;
+        for (int i = lane; i < 16 * MF * nst; i += 64)
+          neg |= reinterpret_cast<const float *>(xs + i / (16 * MF) * Sh::XSB + MF * F::OPS * 1024)[i % (16 * MF)] < 0.f;
+        has_inf = __any(neg);
+      }
+    }
     if (z + NS - 1 < total) issue();  // into the buffer of stage z - 1, which every wave has left
     const char *buf = st0 + cb * Sh::STAGE;
     const char *xb = xs + sbl * Sh::XSB + 16 * lane;
@@ -405,6 +424,34 @@ __global__ void __launch_bounds__(64 * NW) k_rows_mm(const RowsArgs a) {
         float v = F::SCALED ? d * t[m][r] : t[m][r];
         if constexpr (F::MINS) v = fmaf(dm, u[r], v);
         acc[m][r] = fmaf(sc[r], v, acc[m][r]);
+      }
+    }
+    if constexpr (F::MINS) {
+      if (has_inf) {
+        const uint8_t *sb = reinterpret_cast<const uint8_t *>(buf) + row0 * (16 * F::C);
+        const float dmin = half_bits_to_f32(dw[0] >> 16);
+#pragma unroll 1
+        for (int R = 0; R < 16 * MF; ++R) {
+          if (!(reinterpret_cast<const float *>(xsc)[R] < 0.f)) continue;
+          const int64_t e0 = min(R, a.M - 1) * K + (sb0 + sbl) * 256 + 64 * g;
+          float s = 0.f;
+#pragma unroll 1
+          for (int i = 0; i < 64; ++i) {  // this lane's unit
+            const float x = load_elem<XDT>(a.X, e0 + i);
+            if (fabsf(x) < __builtin_inff()) continue;
+            const int h = i >> 5, l = i & 31;
+            uint32_t w = (sb[(FMT == FMT_Q4_K ? 16 : 48) + 32 * g + l] >> (4 * h)) & 15u;
+            if constexpr (FMT == FMT_Q5_K) w |= ((sb[16 + l] >> (2 * g + h)) & 1u) << 4;
+            const float ds = d * static_cast<float>((sc6 >> (8 * h)) & 0xffu), m = dmin * static_cast<float>((mn6 >> (8 * h)) & 0xffu);
+            s += x * fmaf(ds, static_cast<float>(w), -m);
+          }
+          s += __shfl_xor(s, 16, 64);
+          s += __shfl_xor(s, 32, 64);
+#pragma unroll
+          for (int m = 0; m < MF; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[m][r] += R == 16 * m + 4 * g + r ? s : 0.f;
+        }
       }
     }
     cb = cb + 1 < NS ? cb + 1 : 0;
