@@ -49,11 +49,12 @@ def test_rows_gemm(dev, ty, M, N, K):
 
 
 @pytest.mark.parametrize("ty", TYPES)
-@pytest.mark.parametrize("plan,K,splits", [("1,1", 1792, 7), ("2,3", 1792, 4), ("3,2", 1792, 3), ("9,1", 1024, 1)])
+@pytest.mark.parametrize("plan,K,splits", [("1,1", 1792, 7), ("2,3", 1792, 4), ("3,2", 1792, 3), ("9,1", 1024, 1),
+                                           ("1,2,2", 1792, 7), ("3,1,2", 1792, 3), ("2,2,1", 768, 2), ("9,9,2", 1024, 1)])
 def test_rows_gemm_plans(dev, monkeypatch, ty, plan, K, splits):
     """Forced K ranges and workgroups per range: several tiles per workgroup (the LDS stages run on across
-    tiles), a ragged last range, one range (a K whose X fits LDS for every type); f64 output with a residual and a
-    wider row stride."""
+    tiles), a ragged last range, one range (a K whose X fits LDS for every type), rows in groups of 16 and all in one
+    workgroup; f64 output with a residual and a wider row stride."""
     monkeypatch.setenv("VYBDQ_TUNING", "1")
     monkeypatch.setenv("VYBDQ_ROWS_PLAN", plan)
     M, N, ldy = 21, 896, 1000

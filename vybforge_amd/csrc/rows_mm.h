@@ -25,8 +25,8 @@
 // itself streams weights at 4.6 TB/s; the rest is the start (X), the last round of tiles and the
 // reduce (~5 us). Non-finite activations give what the sum over k gives: where the mins are subtracted apart from the
 // products (Q4_K, Q5_K), an infinity would meet zeros and infinities that the weight itself is not, so a row's
-// super-block that holds one is staged as zeros, marked by a negative scale, and its infinities (and NaNs) times their
-// whole weights are added on a path of their own.
+// super-block that holds one is staged as zeros under an infinite scale, and a tile that then holds NaNs takes those rows'
+// infinities (and NaNs) times whole weights instead.
 #pragma once
 #include "gemv_dev.h"
 
@@ -173,7 +173,50 @@ typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 
 template <int XDT> struct RowsX { u4 r[XDT == VYBDQ_F32 ? 2 : 1]; };
 
-template <int FMT, int XDT, int MF, int NW>
+// The rows of a tile whose super-blocks were marked (scale infinite, operands zero: the accumulators of those rows are
+// NaN): their non-finite activations times whole weights, the other terms being finite. All lanes of the wave; column col,
+// unit g, split super-blocks sb0 .. sb0 + nst.
+template <int FMT, int XDT, int MF>
+__device__ __forceinline__ void rows_non_finite(const RowsArgs &a, const char *xs, int sb0, int nst, int m0, int64_t col, int g,
+                                                f4 (&acc)[MF]) {
+  using F = RowsFmt<FMT>;
+  constexpr int XSB = MF * (F::OPS * 1024 + 64);
+#pragma unroll 1
+  for (int R = 0; R < 16 * MF; ++R) {
+    float s = 0.f;
+    bool marked = false;
+#pragma unroll 1
+    for (int b = 0; b < nst; ++b) {
+      if (reinterpret_cast<const float *>(xs + b * XSB + MF * F::OPS * 1024)[R] < __builtin_inff()) continue;
+      marked = true;
+      const uint8_t *sb = a.W + col * a.rowbytes + static_cast<int64_t>(sb0 + b) * F::SBB;
+      const uint32_t *hd = reinterpret_cast<const uint32_t *>(sb);
+      const float d = half_bits_to_f32(hd[0] & 0xffffu), dmin = half_bits_to_f32(hd[0] >> 16);
+      uint32_t sc6, mn6;
+      rows_scales_k4(hd[1], hd[2], hd[3], g, sc6, mn6);
+      const int64_t e0 = (min(m0 + R, a.M - 1) * static_cast<int64_t>(a.SB) + sb0 + b) * 256 + 64 * g;
+#pragma unroll 1
+      for (int i = 0; i < 64; ++i) {
+        const float x = load_elem<XDT>(a.X, e0 + i);
+        if (fabsf(x) < __builtin_inff()) continue;
+        const int h = i >> 5, l = i & 31;
+        uint32_t q = (sb[(FMT == FMT_Q4_K ? 16 : 48) + 32 * g + l] >> (4 * h)) & 15u;
+        if constexpr (FMT == FMT_Q5_K) q |= ((sb[16 + l] >> (2 * g + h)) & 1u) << 4;
+        s += x * fmaf(d * static_cast<float>((sc6 >> (8 * h)) & 0xffu), static_cast<float>(q),
+                      -dmin * static_cast<float>((mn6 >> (8 * h)) & 0xffu));
+      }
+    }
+    if (!marked) continue;
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+#pragma unroll
+    for (int m = 0; m < MF; ++m)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[m][r] = R == 16 * m + 4 * g + r ? s : acc[m][r];
+  }
+}
+
+template <int FMT, int XDT, int MF, int NW, bool GR = false>
 __global__ void __launch_bounds__(64 * NW) k_rows_mm(const RowsArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   using Sh = RowsShape<FMT, MF, NW>;
@@ -181,7 +224,7 @@ __global__ void __launch_bounds__(64 * NW) k_rows_mm(const RowsArgs a) {
   constexpr int PD = Fmt<FMT>::PAIR_DWORDS, PER = Sh::PER;
   const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int sb0 = blockIdx.y * a.sps;
+  const int sb0 = blockIdx.y * a.sps, m0 = GR ? blockIdx.z * 16 * MF : 0;  // K range, first row
   const int nst = min(a.sps, a.SB - sb0), NS = a.ns;
   const int ntile = (a.tiles - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x);
   const int total = ntile * nst;
@@ -190,7 +233,7 @@ __global__ void __launch_bounds__(64 * NW) k_rows_mm(const RowsArgs a) {
   // 1. X of (m-fragment, super-block) task q: lane = row n, 16-byte chunk 4 cc + g of the super-block
   const int64_t K = static_cast<int64_t>(a.SB) * 256;
   auto xload = [&](int q, RowsX<XDT> (&v)[8]) {
-    const int m = q % MF, sb = sb0 + q / MF, row = min(16 * m + n, a.M - 1);
+    const int m = q % MF, sb = sb0 + q / MF, row = min(m0 + 16 * m + n, a.M - 1);
     const int64_t e = row * K + sb * 256 + 8 * g;
 #pragma unroll
     for (int cc = 0; cc < 8; ++cc) {
@@ -226,7 +269,7 @@ __global__ void __launch_bounds__(64 * NW) k_rows_mm(const RowsArgs a) {
     const float sc = block_scale(amax, inv);
     const bool inf = F::MINS && amax == __builtin_inff();
     char *base = xs + (q / MF) * Sh::XSB + (q % MF) * (F::OPS * 1024);
-    if (g == 0) reinterpret_cast<float *>(xs + (q / MF) * Sh::XSB + MF * F::OPS * 1024)[16 * (q % MF) + n] = inf ? -1.0f : sc;
+    if (g == 0) reinterpret_cast<float *>(xs + (q / MF) * Sh::XSB + MF * F::OPS * 1024)[16 * (q % MF) + n] = inf ? amax : sc;
 #pragma unroll
     for (int cc = 0; cc < 8; ++cc) {  // block cc of the super-block; this lane's chunk: quarter g
       u4 o;
@@ -360,18 +403,9 @@ __global__ void __launch_bounds__(64 * NW) k_rows_mm(const RowsArgs a) {
   for (int m = 0; m < MF; ++m) acc[m] = f4{0.f, 0.f, 0.f, 0.f};
   const int row0 = wave * 16 + n;  // this lane's weight row within the tile
   int tile = blockIdx.x, sbl = 0, cb = 0;
-  bool has_inf = false;  // a marked super-block among the workgroup's
   for (int z = 0; z < total; ++z) {
     wait_later(min(NS - 2, total - 1 - z));
     bar();
-    if constexpr (F::MINS) {
-      if (z == 0) {
-        bool neg = false;
-        for (int i = lane; i < 16 * MF * nst; i += 64)
-          neg |= reinterpret_cast<const float *>(xs + i / (16 * MF) * Sh::XSB + MF * F::OPS * 1024)[i % (16 * MF)] < 0.f;
-        has_inf = __any(neg);
-      }
-    }
     if (z + NS - 1 < total) issue();  // into the buffer of stage z - 1, which every wave has left
     const char *buf = st0 + cb * Sh::STAGE;
     const char *xb = xs + sbl * Sh::XSB + 16 * lane;
@@ -426,43 +460,23 @@ __global__ void __launch_bounds__(64 * NW) k_rows_mm(const RowsArgs a) {
         acc[m][r] = fmaf(sc[r], v, acc[m][r]);
       }
     }
-    if constexpr (F::MINS) {
-      if (has_inf) {
-        const uint8_t *sb = reinterpret_cast<const uint8_t *>(buf) + row0 * (16 * F::C);
-        const float dmin = half_bits_to_f32(dw[0] >> 16);
-#pragma unroll 1
-        for (int R = 0; R < 16 * MF; ++R) {
-          if (!(reinterpret_cast<const float *>(xsc)[R] < 0.f)) continue;
-          const int64_t e0 = min(R, a.M - 1) * K + (sb0 + sbl) * 256 + 64 * g;
-          float s = 0.f;
-#pragma unroll 1
-          for (int i = 0; i < 64; ++i) {  // this lane's unit
-            const float x = load_elem<XDT>(a.X, e0 + i);
-            if (fabsf(x) < __builtin_inff()) continue;
-            const int h = i >> 5, l = i & 31;
-            uint32_t w = (sb[(FMT == FMT_Q4_K ? 16 : 48) + 32 * g + l] >> (4 * h)) & 15u;
-            if constexpr (FMT == FMT_Q5_K) w |= ((sb[16 + l] >> (2 * g + h)) & 1u) << 4;
-            const float ds = d * static_cast<float>((sc6 >> (8 * h)) & 0xffu), m = dmin * static_cast<float>((mn6 >> (8 * h)) & 0xffu);
-            s += x * fmaf(ds, static_cast<float>(w), -m);
-          }
-          s += __shfl_xor(s, 16, 64);
-          s += __shfl_xor(s, 32, 64);
-#pragma unroll
-          for (int m = 0; m < MF; ++m)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[m][r] += R == 16 * m + 4 * g + r ? s : 0.f;
-        }
-      }
-    }
     cb = cb + 1 < NS ? cb + 1 : 0;
     if (++sbl < nst) continue;
-    // acc[m][r] = C[16 m + 4 g + r][BN tile + row0]
+    // acc[m][r] = C[m0 + 16 m + 4 g + r][BN tile + row0]
     const int64_t col = static_cast<int64_t>(tile) * Sh::BN + row0;
+    if constexpr (F::MINS) {
+      bool nan = false;
+#pragma unroll
+      for (int m = 0; m < MF; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) nan |= acc[m][r] != acc[m][r];
+      if (__any(nan)) rows_non_finite<FMT, XDT, MF>(a, xs, sb0, nst, m0, col, g, acc);
+    }
 #pragma unroll
     for (int m = 0; m < MF; ++m) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = 16 * m + 4 * g + r;
+        const int row = m0 + 16 * m + 4 * g + r;
         if (row >= a.M) continue;
         if (a.splits > 1) {
           a.part[(static_cast<int64_t>(blockIdx.y) * a.M + row) * a.N + col] = acc[m][r];

@@ -32,7 +32,9 @@ __global__ void __launch_bounds__(256) k_rows_reduce(const RowsArgs a) {
 }
 
 struct RowsPlan {
-  int NW, splits, sps, nwg, ns;  // waves (16 weight rows each), K splits, super-blocks per split, workgroups per split, stages
+  // waves (16 weight rows each), K splits, super-blocks per split, workgroups per split and row group, stages, X row
+  // fragments per workgroup, row groups
+  int NW, splits, sps, nwg, ns, MF, groups;
 };
 
 // 16 waves (256 weight rows a tile) up to 32 X rows: with 8 (two per SIMD) a wave's decode waits on its
@@ -40,21 +42,30 @@ struct RowsPlan {
 // need the registers of 8 waves; and so may LDS (Q8_0: two stages of 256 rows and one X super-block are all
 // of it). One workgroup fits a CU; the plan minimises the stages of the busiest CU (a stage's bytes at
 // the 18.5 GB/s a CU gets of HBM) plus a workgroup's start (X staging) and the split partials, written
-// and read back. With only two LDS stages a stage is barely in flight: 10% more. Only plans whose partials
-// fit ws_bytes are looked at. VYBDQ_ROWS_PLAN="sps,nwg" overrides the split (ignored where it does not fit).
+// and read back. With only two LDS stages a stage is barely in flight: 10% more.
+// Up to 2^22 weights the chip is idle and a workgroup's own chain counts, which grows with its X rows (LDS reads of the
+// operands, staging): every 16 rows get workgroups of their own (W again from L2), of 8 waves (twice the workgroups of 16), and a
+// stage costs its latency.
+// 64 rows, X all in one workgroup / in groups of 16: 512 x 512 q4_0 9.4 / 5.5 us, Q4_K 11.8 / 6.4, IQ2_S 10.8 / 7.3; 1024 x
+// 1024 8.2 / 6.7, 10.1 / 7.7, 9.2 / 7.9; 2048 x 2048 10.6 / 9.3, 12.4 / 10.2, 10.9 / 10.6; 2560 x 2560 12.8 / 12.0, 14.5 / 12.6 but IQ2_S
+// 14.1 / 14.2 (its decode is repeated per group). (The unscaled tiles of the calls without a workspace: 512 x 512 5.3, 7.9, 8.7;
+// Q8_0, whose decode is short, 5.2 against 5.9 here.) Only plans whose partials
+// fit ws_bytes are looked at. VYBDQ_ROWS_PLAN="sps,nwg[,groups]" overrides
+// the split (and whether rows are grouped: 1 or more); ignored where it does not fit.
 template <int FMT>
 static RowsPlan rows_plan(int M, int64_t N, int64_t K, int64_t ws_bytes) {
   using F = RowsFmt<FMT>;
-  const int SB = static_cast<int>(K / 256), MF = (M + 15) / 16, cus = 256;
-  const int xsb = MF * (F::OPS * 1024 + 64), tab = FMT == FMT_IQ2_S ? kRowsGrid : 0;
+  const int SB = static_cast<int>(K / 256), MT = (M + 15) / 16, cus = 256, tab = FMT == FMT_IQ2_S ? kRowsGrid : 0;
   RowsPlan best{};
   double best_t = -1;
-  int fs = 0, fn = 0;
+  int fs = 0, fn = 0, fg = 0;
   if (const char *e = tuning_env("VYBDQ_ROWS_PLAN"))
-    if (sscanf(e, "%d,%d", &fs, &fn) != 2 || fs < 1 || fn < 1) fs = fn = 0;
+    if (sscanf(e, "%d,%d,%d", &fs, &fn, &fg) < 2 || fs < 1 || fn < 1) fs = fn = fg = 0;
   if (fs > SB) fs = SB;
-  for (;; fs = 0) {
-    for (int NW = MF <= 2 ? 16 : 8; NW >= 4; NW /= 2) {
+  for (;; fs = fg = 0) {
+    const bool small = fg ? fg > 1 : MT > 1 && N * K <= (1 << 22);
+    const int groups = small ? MT : 1, MF = MT / groups, xsb = MF * (F::OPS * 1024 + 64);
+    for (int NW = MF <= 2 && !small ? 16 : 8; NW >= 4; NW /= 2) {
       const int BN = 16 * NW, tiles = static_cast<int>(N / BN), stage = BN * F::C * 16;
       if (N % BN || (NW == 4 && N % 128 == 0)) continue;  // 4 waves only where 8 do not divide N
       for (int sps = fs ? fs : 1; sps <= SB && sps <= (fs ? fs : 32); ++sps) {
@@ -63,16 +74,23 @@ static RowsPlan rows_plan(int M, int64_t N, int64_t K, int64_t ws_bytes) {
         if (ns < 2) break;
         ns = ns > 4 ? 4 : ns;
         if (splits > kRowsMaxSplits || (splits > 1 && splits * M * N * 4 > ws_bytes)) continue;
-        int nwg = cus / splits > 0 ? cus / splits : 1;
+        int nwg = cus / (splits * groups) > 0 ? cus / (splits * groups) : 1;
         if (fs) nwg = fn;
         nwg = nwg < tiles ? nwg : tiles;
-        const int rounds = (splits * nwg + cus - 1) / cus, stages = (tiles + nwg - 1) / nwg * sps;
-        double t = rounds * (stages * stage / 18.5e3 * (ns == 2 ? 1.1 : 1.0) + 2.5 + 0.2 * sps * MF);
-        if (NW < 16 && MF <= 2) t *= 1.08;
-        if (splits > 1) t += 4.0 + 8.0 * splits * M * static_cast<double>(N) / 4.0e6;
+        const int wgs = splits * groups * nwg, rounds = (wgs + cus - 1) / cus, stages = (tiles + nwg - 1) / nwg * sps;
+        const double part = splits * M * static_cast<double>(N) / 1.0e6;
+        double t;
+        if (small) {
+          t = rounds * stages * (FMT == FMT_Q6_K || FMT == FMT_IQ2_S ? 1.85 : 1.2) + static_cast<double>(wgs) / cus;
+          if (splits > 1) t += 2.0 + 1.5 * part;
+        } else {
+          t = rounds * (stages * stage / 18.5e3 * (ns == 2 ? 1.1 : 1.0) + 2.5 + 0.2 * sps * MF);
+          if (NW < 16 && MF <= 2) t *= 1.08;
+          if (splits > 1) t += 4.0 + 2.0 * part;
+        }
         if (best_t < 0 || t < best_t) {
           best_t = t;
-          best = {NW, splits, sps, nwg, ns};
+          best = {NW, splits, sps, nwg, ns, MF, groups};
         }
       }
     }
@@ -111,21 +129,24 @@ int64_t rows_mm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
   return need;
 }
 
-template <int FMT, int XDT, int MF, int NW>
+template <int FMT, int XDT, int MF, int NW, bool GR = false>
 static int rows_launch(const RowsArgs &a, const RowsPlan &p, hipStream_t s) {
   using Sh = RowsShape<FMT, MF, NW>;
   static std::atomic<uint64_t> raised{0};
-  const int rc = ensure_lds_limit(reinterpret_cast<const void *>(&k_rows_mm<FMT, XDT, MF, NW>), 160 * 1024, raised,
+  const int rc = ensure_lds_limit(reinterpret_cast<const void *>(&k_rows_mm<FMT, XDT, MF, NW, GR>), 160 * 1024, raised,
                                   "gemm (few rows)");
   if (rc) return rc;
   const size_t lds = Sh::TAB + static_cast<size_t>(p.sps) * Sh::XSB + static_cast<size_t>(p.ns) * Sh::STAGE;
-  hipLaunchKernelGGL((k_rows_mm<FMT, XDT, MF, NW>), dim3(static_cast<unsigned>(p.nwg), static_cast<unsigned>(p.splits)),
-                     dim3(64 * NW), lds, s, a);
+  hipLaunchKernelGGL((k_rows_mm<FMT, XDT, MF, NW, GR>), dim3(static_cast<unsigned>(p.nwg), static_cast<unsigned>(p.splits),
+                     static_cast<unsigned>(p.groups)), dim3(64 * NW), lds, s, a);
   return check_launch("gemm (few rows)");
 }
 
 template <int FMT, int XDT, int MF>
 static int rows_launch_p(const RowsArgs &a, const RowsPlan &p, hipStream_t s) {
+  if constexpr (MF == 1) {
+    if (p.groups > 1) return p.NW == 8 ? rows_launch<FMT, XDT, 1, 8, true>(a, p, s) : rows_launch<FMT, XDT, 1, 4, true>(a, p, s);
+  }
   if constexpr (MF <= 2) {
     if (p.NW == 16) return rows_launch<FMT, XDT, MF, 16>(a, p, s);
   }
@@ -135,7 +156,7 @@ static int rows_launch_p(const RowsArgs &a, const RowsPlan &p, hipStream_t s) {
 
 template <int FMT, int XDT>
 static int rows_launch_x(const RowsArgs &a, const RowsPlan &p, hipStream_t s) {
-  switch ((a.M + 15) / 16) {
+  switch (p.MF) {
     case 1: return rows_launch_p<FMT, XDT, 1>(a, p, s);
     case 2: return rows_launch_p<FMT, XDT, 2>(a, p, s);
     case 3: return rows_launch_p<FMT, XDT, 3>(a, p, s);
