@@ -29,9 +29,10 @@ def test_rmsnorm_q8(dev, xdt, M, N):
     np.testing.assert_array_equal(Xs.cpu().numpy(), d)
 
 
-@pytest.mark.parametrize("M,N", [(1, 288), (5, 2592), (200, 544), (511, 256), (600, 1056)])
+@pytest.mark.parametrize("M,N", [(1, 288), (5, 2592), (200, 544), (511, 256), (600, 1056), (256, 256), (257, 2048),
+                                 (257, 2080)])
 def test_rmsnorm_q8_row_parts(dev, M, N):
-    """Rows split over workgroups (ragged last part, several 256-column chunks per part, unsplit) and the same rows
+    """Rows split over workgroups (ragged last part, several 256-column chunks per part), unsplit rows on either side of the rule, and the same rows
     written over their input (Y and X one buffer: the unsplit kernel): bit-equal to the oracle."""
     rng = np.random.default_rng(M + N)
     x = torch.from_numpy(rng.standard_normal((M, N)).astype(np.float32))

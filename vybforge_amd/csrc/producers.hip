@@ -284,7 +284,10 @@ extern "C" int vybdq_rmsnorm_q8(uint64_t X, uint64_t W, uint64_t Y, uint64_t Y32
   // row; measured, float32 5120 columns: 1 row 14.8 -> 6.0 us with a SwiGLU launch beside it, 64 rows
   // 15.9 -> 8.5 (8 parts; 20 parts 9.1), 512 rows 23.6 -> 23.1 unsplit, 40 in 20 parts). Outputs over the
   // inputs need the row in registers before the first store, and float64 rows unsplit are faster that way
-  // (512 rows 23.2 us against 24.7): the one-workgroup kernel.
+  // (512 rows 23.2 us against 24.7): the one-workgroup kernel. So are short rows that come in numbers, where its row is
+  // a few registers and one pass: float32 2000 x 1024 7.4 us against 9.4, 2000 x 2048 12.0 / 13.7, 512 x 1024 4.9 / 5.2 (but
+  // 2000 x 2560 21.0 / 17.0 here, 256 x 256 the same), rows of about 4096 that fill its registers up to some 1500 of
+  // them (bf16 1000 x 4096 14.6 / 15.3, 2000 x 4096 25.6 / 23.9), and float64 256 x 768 by 8% even where the split would be two.
   auto overlaps = [](uint64_t o, int64_t ob, uint64_t i, int64_t ib) {
     return o && o < i + static_cast<uint64_t>(ib) && i < o + static_cast<uint64_t>(ob);
   };
@@ -296,7 +299,9 @@ extern "C" int vybdq_rmsnorm_q8(uint64_t X, uint64_t W, uint64_t Y, uint64_t Y32
   const int64_t chunks = (N + 255) / 256, want = M < 512 ? 512 / M : 1;
   const int64_t E = (chunks + (want < chunks ? want : chunks) - 1) / (want < chunks ? want : chunks) * 256;
   const unsigned parts = static_cast<unsigned>((N + E - 1) / E);
-  if (!alias && (parts > 1 || x_dt != VYBDQ_F64) && M < 65536) {
+  const bool long_row = N > 2048 && (N <= 3072 || N > 4096 || M > 1500);
+  const bool split = parts > 1 ? x_dt != VYBDQ_F64 || N > 1024 || M <= 128 : x_dt != VYBDQ_F64 && (long_row || M <= 256);
+  if (!alias && split && M < 65536) {
     VYBDQ_DISPATCH_ANY(x_dt, XDT, hipLaunchKernelGGL((k_rms_q8_parts<XDT>), dim3(parts, static_cast<unsigned>(M)),
                                                      dim3(256), 0, s, x, w, y, y_dt, y32, q, d, N, E, eps));
     return check_launch("vybdq_rmsnorm_q8");
