@@ -39,6 +39,20 @@ def test_gemv_xq8_matches_gate(dev, ty, N, K):
 
 
 @pytest.mark.parametrize("ty", TYPES)
+@pytest.mark.parametrize("plan,N,K", [("8,1,256", 77, 512), ("8,2,256", 300, 1280), ("16,1,64", 50, 2304), ("16,3,256", 130, 3328),
+                                      ("32,1,128", 64, 9728), ("64,2,256", 36, 8448), ("64,4,256", 5, 17408),
+                                      (None, 32768, 256), (None, 1024, 4352), (None, 1025, 4352)])
+def test_gemv_xq8_plans(dev, monkeypatch, ty, plan, N, K):
+    """Lanes per row and windows per lane forced (units that do not fill the last window, idle lanes), and the sizes at
+    which the planner turns from one window per lane to several."""
+    if plan:
+        monkeypatch.setenv("VYBDQ_GEMV_PLAN", plan)
+    raw, x, W, xq, xd = _setup(dev, ty, N, K, seed=N + K + ty)
+    y = ops.gemv_xq8(ty, W, xq, xd, N, K).cpu().numpy()
+    assert matmul.rel_maxnorm(y, matmul.gemv_xq8_f64(ty, raw, xq.cpu().numpy(), xd.cpu().numpy(), N, K)) < XQ8_TOL
+
+
+@pytest.mark.parametrize("ty", TYPES)
 def test_gemv_xq8_against_the_exact_gemv(dev, ty):
     # lossy by the activation quantization only: the exact GEMV of x differs by well under 2%
     N, K = 2048, 4096

@@ -16,8 +16,8 @@
 //     sign byte, d (0.5 + s) / 4 per 16 weights with the 4-bit scales s.
 //
 // Work split and loads as the exact pair GEMV (gemv_pair.h): G lanes per row walk its 64-weight
-// units with stride G, one unit window at a time (load_unit_kq), the first issued before x is
-// staged, partial sums combined by the DPP tree. LDS holds, per unit p, the 64 xq
+// units with stride G, U unit windows in flight per lane (load_unit_kq; one on most grids, xq8_plan), the first issued
+// before x is staged, partial sums combined by the DPP tree. LDS holds, per unit p, the 64 xq
 // bytes at 80 p (16 bytes of padding put the G lanes reading consecutive units on distinct banks:
 // a lane reads its unit's x with four conflict-free ds_read_b128) and float4 {dx, sum(xq)} x 2 of
 // its two blocks; IQ2_S adds the grid as bytes (1024 x 8 B) and the 256 sign patterns as byte
@@ -99,7 +99,7 @@ __device__ __forceinline__ float unit_dot_xq8(const uint32_t (&dw)[Fmt<FMT>::PAI
   }
 }
 
-template <int FMT, int G>
+template <int FMT, int G, int U>
 __global__ void __launch_bounds__(256) k_gemv_xq8(const int8_t *__restrict__ Xq, const float *__restrict__ Xs,
                                                   int64_t K, Segs segs) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -130,9 +130,10 @@ __global__ void __launch_bounds__(256) k_gemv_xq8(const int8_t *__restrict__ Xq,
     return p < P ? p : (ks < P ? ks : 0);
   };
 
-  // 1. the first weight window
-  uint32_t dw[PD];
-  load_unit_kq<FMT>(wrow, unit_idx(0), dw);
+  // 1. the first U weight windows
+  uint32_t dw[U][PD];
+#pragma unroll
+  for (int u = 0; u < U; ++u) load_unit_kq<FMT>(wrow, unit_idx(u), dw[u]);
 
   // 2. x -> LDS under those loads: 16-byte chunks of xq (chunk c = bytes 16c .. 16c+15, block c / 2,
   // unit c / 4) with the block sums by one DPP swap between the chunk pair's two threads (K / 16 is
@@ -165,9 +166,14 @@ __global__ void __launch_bounds__(256) k_gemv_xq8(const int8_t *__restrict__ Xq,
   __syncthreads();
 
   float acc = 0.f;
-  for (int i = 0; i < nunits; ++i) {
-    if (i > 0) load_unit_kq<FMT>(wrow, unit_idx(i), dw);
-    acc += unit_dot_xq8<FMT>(dw, lq, lmeta, lgrid, lsign, ks + G * i);
+  for (int i0 = 0; i0 < nunits; i0 += U) {
+    if (i0 > 0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) load_unit_kq<FMT>(wrow, unit_idx(i0 + u), dw[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i0 + u < nunits) acc += unit_dot_xq8<FMT>(dw[u], lq, lmeta, lgrid, lsign, ks + G * (i0 + u));
   }
   acc = group_sum<G>(acc);
   if (active && ks == G - 1) {
@@ -182,32 +188,53 @@ __global__ void __launch_bounds__(256) k_gemv_xq8(const int8_t *__restrict__ Xq,
   }
 }
 
-template <int FMT, int G>
-static int xq8_launch_g(const int8_t *Xq, const float *Xs, int64_t K, const Segs &segs, int threads, hipStream_t s) {
+template <int FMT, int G, int U>
+static int xq8_launch_gu(const int8_t *Xq, const float *Xs, int64_t K, const Segs &segs, int threads, hipStream_t s) {
   const int64_t P = K / 64;
   const size_t lds = xq8_lds_bytes(P, FMT == FMT_IQ2_S);
   if (lds > static_cast<size_t>(kMaxLds)) return set_error(VYBDQ_ERR_SHAPE, "gemv_xq8: K too large for the LDS x stage");
   if (lds > 64 * 1024) {
     static std::atomic<uint64_t> raised{0};
-    const int rc = ensure_lds_limit(reinterpret_cast<const void *>(&k_gemv_xq8<FMT, G>), kMaxLds, raised, "gemv_xq8");
+    const int rc = ensure_lds_limit(reinterpret_cast<const void *>(&k_gemv_xq8<FMT, G, U>), kMaxLds, raised, "gemv_xq8");
     if (rc) return rc;
   }
   const int rows_per_wg = threads / G;
   const unsigned grid = static_cast<unsigned>((segs.end[2] + rows_per_wg - 1) / rows_per_wg);
-  hipLaunchKernelGGL((k_gemv_xq8<FMT, G>), dim3(grid), dim3(threads), lds, s, Xq, Xs, K, segs);
+  hipLaunchKernelGGL((k_gemv_xq8<FMT, G, U>), dim3(grid), dim3(threads), lds, s, Xq, Xs, K, segs);
   return check_launch("gemv_xq8");
 }
 
-// Lanes per row: one unit window in flight per lane and many waves instead of the exact GEMV's batches
-// (the integer dot holds more registers than it needs: 8 waves per SIMD against 5), so G only has to keep
-// a row's units even over the lanes: 16 up to 128 units (K = 8192), 32 above, more while the grid has fewer
-// than two workgroups per CU (Q4_K 2560 x 9728: G = 64 6.5 us, 32 7.3). Measured, one window against the exact GEMV's plan: two 17408 x 5120 matrices IQ2_S
-// 19.7 us at G = 16 (22.8), Q4_K 22.7 (24.0), Q5_K 26.1 (28.0); 5120 x 17408 at G = 32: IQ2_S 15.3 us
-// (17.6), Q4_K 13.2 (14.9), Q5_K 15.0 (15.5); at G = 16 19.9, 14.9 and 17.5.
+template <int FMT, int G>
+static int xq8_launch_g(const int8_t *Xq, const float *Xs, int64_t K, const Segs &segs, const PairPlan &pl,
+                        hipStream_t s) {
+  constexpr int UM = kUmax<FMT>();
+  switch (pl.U) {
+    case 1: return xq8_launch_gu<FMT, G, 1>(Xq, Xs, K, segs, pl.T, s);
+    case 2: return xq8_launch_gu<FMT, G, 2>(Xq, Xs, K, segs, pl.T, s);
+    case 3: return xq8_launch_gu<FMT, G, (UM < 3 ? UM : 3)>(Xq, Xs, K, segs, pl.T, s);
+    default: return xq8_launch_gu<FMT, G, UM>(Xq, Xs, K, segs, pl.T, s);
+  }
+}
+
+// Lanes per row and unit windows in flight per lane. Where several workgroups share a CU, one window per lane and many
+// waves (the integer dot holds more registers than it needs: 8 waves per SIMD against 5 of the exact GEMV's plan), and G
+// only has to keep a row's units even over the lanes: 8 up to 8 units (K = 512), 16 up to 120, 32 above, more while a row
+// has more units than lanes and the grid fewer than two workgroups per CU (Q4_K 2560 x 9728: G = 64 6.5 us, 32 7.3). Measured,
+// one window against the exact GEMV's plan: two 17408 x 5120 matrices IQ2_S 19.7 us (22.8), Q4_K 22.7 (24.0), Q5_K 26.1
+// (28.0); 5120 x 17408 at G = 32: IQ2_S 15.3 us (17.6), Q4_K 13.2 (14.9), Q5_K 15.0 (15.5); at G = 16 19.9, 14.9 and 17.5.
+// The exact GEMV's plan, several windows per lane, where that measured faster: a grid of at most one workgroup per CU at 64
+// lanes (Q4_K 768 x 9728 4.7 us against 5.1, 256 x 25600 6.8 / 7.9), and many rows of few units, where every workgroup
+// stages x for little work (151936 rows: IQ2_S K = 256 12.7 / 21.1, Q4_K K = 1024 17.7 / 20.8, K = 2048 30.0 / 30.9).
+// A long x lets only some workgroups into a CU's LDS: a grid just past one round of those takes half the lanes (Q4_K
+// 9728 x 25600, four to a CU: G = 32 37.8 us, 16 32.5).
 static PairPlan xq8_plan(int fmt, int64_t rows, int P) {
-  PairPlan pl{P <= 128 ? 16 : 32, 1, 256};
-  while (pl.G < 64 && rows * pl.G / 256 < 2 * device_cu_count()) pl.G *= 2;
-  if (tuning_env("VYBDQ_GEMV_PLAN")) pl = pair_plan(fmt, rows, P, 1);  // the override's G and T
+  const int64_t cus = device_cu_count();
+  if ((P > 64 && rows * 64 <= 256 * cus) || (P <= 32 && rows >= 128 * cus) || tuning_env("VYBDQ_GEMV_PLAN"))
+    return pair_plan(fmt, rows, P, 1);
+  PairPlan pl{P <= 8 ? 8 : P <= 120 ? 16 : 32, 1, 256};
+  while (pl.G < 64 && P > pl.G && rows * pl.G / 256 < 2 * cus) pl.G *= 2;
+  const int64_t per_cu = kMaxLds / static_cast<int64_t>(xq8_lds_bytes(P, fmt == FMT_IQ2_S)), wgs = rows * pl.G / 256;
+  if (per_cu < 8 && pl.G > 16 && wgs > per_cu * cus && 4 * wgs < 5 * per_cu * cus) pl.G /= 2;
   return pl;
 }
 
@@ -215,10 +242,10 @@ template <int FMT>
 static int xq8_launch(const int8_t *Xq, const float *Xs, int64_t K, const Segs &segs, hipStream_t s) {
   const PairPlan pl = xq8_plan(FMT, segs.end[2], static_cast<int>(K / 64));
   switch (pl.G) {
-    case 8: return xq8_launch_g<FMT, 8>(Xq, Xs, K, segs, pl.T, s);
-    case 16: return xq8_launch_g<FMT, 16>(Xq, Xs, K, segs, pl.T, s);
-    case 32: return xq8_launch_g<FMT, 32>(Xq, Xs, K, segs, pl.T, s);
-    default: return xq8_launch_g<FMT, 64>(Xq, Xs, K, segs, pl.T, s);
+    case 8: return xq8_launch_g<FMT, 8>(Xq, Xs, K, segs, pl, s);
+    case 16: return xq8_launch_g<FMT, 16>(Xq, Xs, K, segs, pl, s);
+    case 32: return xq8_launch_g<FMT, 32>(Xq, Xs, K, segs, pl, s);
+    default: return xq8_launch_g<FMT, 64>(Xq, Xs, K, segs, pl, s);
   }
 }
 
