@@ -61,3 +61,15 @@ def test_moe_exl3_size_covers_fewer_tokens():
             for k in (1, 4, 8):
                 sizes = [f(T, H, I, E, k) for T in Ts]
                 assert sizes == sorted(sizes), (H, I, E, k)
+
+
+@pytest.mark.parametrize("B", [1, 2, 4, 16])
+def test_exl3_splits_feed_every_wave(B):
+    """Four waves of a workgroup take 64 k at a time: from K = 512 no split is planned that leaves some idle."""
+    for K in (512, 1024, 1536, 1920, 2048, 4096, 5120):
+        for N in (768, 1536, 2048, 5120, 9728, 14848, 17408):
+            arrivals = (N // 128 * 4 + 255) // 256 * 256
+            rotated = 0 if B <= 2 else (B * K * 2 + 255) // 256 * 256
+            size = _lib.lib.vybdq_exl3_workspace_size(B, K, N)
+            own = [s for s in range(1, 17) if arrivals + rotated + s * B * N * 4 <= size]
+            assert max(own) <= -(-K // 256) or B > 2, (K, N)  # (above 2 rows the size covers batches of 2 as well)

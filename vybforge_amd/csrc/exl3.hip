@@ -319,9 +319,10 @@ static int exl3_bp(int64_t B) { return B <= 1 ? 1 : B <= 2 ? 2 : B <= 4 ? 4 : B 
 
 // K-splits: whole 128 chunks (the x rotation is done per chunk), and from 256 k on a multiple of 256
 // k, one 64-k step for each of the four waves. The product is bound by the decode on the VALU, so the
-// time follows the k-blocks that the fullest CU decodes: ceil(workgroups / CUs) * kbs, plus a little per
-// workgroup, per k-block of x rotated before the first step (batch <= 2) and per split of partials written
-// and read back (larger batches). Measured, batch 16: K = 5120, N = 17408: 5 splits (3 workgroups of
+// time follows the k-blocks that the fullest CU decodes: ceil(workgroups / CUs) * kbs (at batch <= 2, 8 k-blocks cost as
+// 16: two of the waves idle), plus a little per workgroup, per k-block of x rotated before the first step (batch <= 2) and per split of
+// partials written and read back, which at batch <= 2 the last arrival reads alone (K = 2048, N = 5120, batch 1: 4 splits
+// of 32 k-blocks 7.7 us, 8 of 16 8.2, 16 of 8 10.6; K = 4096, N = 1536: 8 splits 8.2, 16 9.4). Measured, batch 16: K = 5120, N = 17408: 5 splits (3 workgroups of
 // 64 k-blocks a CU) 25.8 us per call, 4 (3 x 80) 27.5, 7 (4 x 48) 26.2, 10 (6 x 32) 27.3; K = 17408, N = 5120:
 // 12 (2 x 96) 26.6, 17 (3 x 64) 28.1, 10 (2 x 112) 28.2, 14 (3 x 80) 29.6; K = 9216, N = 3072: 9 (1 x 64)
 // 17.6, 12 (2 x 48) 20.0. Batch 1, K = 17408: 12 splits 22.6, 10 24.4, 7 27.3 us.
@@ -342,8 +343,8 @@ static Exl3Split exl3_splits(int64_t K, int64_t N, int BP) {
   for (int S = 1; S <= 16; ++S) {
     const Exl3Split c = shape(S);
     if (exl3_lds_bytes(BP, c.kbs) > kExl3MaxLds) continue;
-    const int64_t rounds = (groups * c.S + 255) / 256;
-    const int64_t cost = exl3_fused(BP) ? rounds * (8 * c.kbs + 16) + BP * c.kbs : rounds * (8 * c.kbs + 48) + 8 * c.S;
+    const int64_t rounds = (groups * c.S + 255) / 256, steps = 8 * (c.kbs > 16 ? c.kbs : 16);
+    const int64_t cost = exl3_fused(BP) ? rounds * (steps + 8) + 3 * BP * c.kbs + 32 * c.S : rounds * (8 * c.kbs + 48) + 8 * c.S;
     if (best_cost < 0 || cost < best_cost) best_cost = cost, best = c;
   }
   if (const char *e = tuning_env("VYBDQ_EXL3_SPLITS")) {  // tuning override
