@@ -779,6 +779,7 @@ __global__ void __launch_bounds__(256) k_kq_reduce(const float *__restrict__ par
 struct Kq2Plan {
   int m_tiles, n_tiles, splits, sps;
   int64_t part_bytes;
+  double us;  // the estimate
 };
 
 // K split minimising the busiest CU's time plus the partial traffic (written once, read back
@@ -788,7 +789,7 @@ struct Kq2Plan {
 static Kq2Plan kq2_plan(int M, int N, int S2, bool allow_split) {
   const int cus = device_cu_count();
   const int m_tiles = (M + kK2BM - 1) / kK2BM, n_tiles = N / kK2BN;
-  Kq2Plan best{m_tiles, n_tiles, 1, S2, 0};
+  Kq2Plan best{m_tiles, n_tiles, 1, S2, 0, 0.0};
   double best_t = -1;
   for (int splits = 1; splits <= (allow_split ? 8 : 1) && splits <= S2; ++splits) {
     const int sps = (S2 + splits - 1) / splits;
@@ -799,7 +800,7 @@ static Kq2Plan kq2_plan(int M, int N, int S2, bool allow_split) {
     double t = sps * (static_cast<double>(c / 3) * 2.98 + rem);
     if (splits > 1) t += static_cast<double>(M) * N * 4 * (splits + 1) / 5.0e6 + 3.0;
     if (best_t < 0 || t < best_t - 1e-9) {
-      best_t = t;
+      best_t = best.us = t;
       best.splits = splits;
       best.sps = sps;
     }
@@ -820,6 +821,10 @@ static Kq2Plan kq2_plan(int M, int N, int S2, bool allow_split) {
 }
 
 static int64_t kq_align256(int64_t b) { return (b + 255) / 256 * 256; }
+
+double kq2_plan_us(int64_t M, int64_t N, int64_t K) {
+  return kq2_plan(static_cast<int>(M), static_cast<int>(N), static_cast<int>(K / 128), true).us;
+}
 
 // 32-bit byte offsets: X (M K fp16), a weight tile (64 rows)
 bool kq2_supported(int wtype, int64_t M, int64_t N, int64_t K) {

@@ -23,6 +23,7 @@ extern template int mmq_launch<FMT_Q5_K, VYBDQ_F16>(MmArgs &, hipStream_t);
 struct MmPlan {
   int m_tiles, n_tiles, F, splits, sps;
   int64_t ws_bytes;  // partials + counters (0 without split-K)
+  double us;         // the estimate
 };
 
 static int64_t mm_part_bytes(int64_t tiles, int splits) {
@@ -60,7 +61,7 @@ static MmPlan mm_plan(int M, int N, int S, bool allow_split, int nfx = kMmNFX, d
         t += bytes / 2.5e6;  // written, then read back by the reducing workgroups
       }
       if (best_t < 0 || t < best_t - 1e-9) {
-        best_t = t;
+        best_t = best.us = t;
         best.m_tiles = m_tiles;
         best.n_tiles = n_tiles;
         best.F = F;
@@ -129,6 +130,12 @@ static int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 // Q4_K / Q5_K tiles: at most 16 fragments (two per wave: its nibble windows, the scale words and
 // 96 accumulators fill the 256 registers of a wave at three)
 static int mm_nfx(int wtype) { return wtype == 12 || wtype == 13 ? 4 : kMmNFX; }
+
+// the planner's estimate of a call with its workspace, in its own microseconds (what it leaves out is the same for
+// every plan of the call)
+double mmq_plan_us(int wtype, int64_t M, int64_t N, int64_t K) {
+  return mm_plan(static_cast<int>(M), static_cast<int>(N), static_cast<int>(K / 128), true, mm_nfx(wtype)).us;
+}
 
 int64_t mmq_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
   if (!mmq_supported(M, N, K)) return 0;

@@ -220,48 +220,64 @@ __global__ void __launch_bounds__(512, 2) k_wide_mm(const WideArgs a) {
 
 static int64_t wide_align256(int64_t b) { return (b + 255) / 256 * 256; }
 
-// Row fragments of 64 per tile (2, 3 or 4), or 0 where the fused bodies are the better choice: the estimate of
-// this path (expand at 5 TB/s; rounds of 256 tiles at the measured time of a K step, which grows with the share
-// of CUs at work) has to be 8% below the fused body's time at the type's rate. Measured, both sides, bf16 X:
-// 1999 rows 17408 x 5120 q4_0 447 us against 496 fused, Q8_0 468 / 535, Q4_K 465 / 542, Q5_K 462 / 600, Q6_K 466 / 633,
-// IQ2_S 471 / 632; 5120 x 17408 (fewer tiles) q4_0 456 / 383, Q4_K 466 / 488, Q6_K 477 / 654; 512 rows 17408 x 5120 q4_0
-// 166 / 113, Q4_K 179 / 157, Q6_K 177 / 207; 1400 rows 17408 x 5120 Q4_K 358 / 349, Q6_K 359 / 462. At most 2^29
-// weights (1 GiB of workspace).
+double mmq_plan_us(int wtype, int64_t M, int64_t N, int64_t K);
+double kq2_plan_us(int64_t M, int64_t N, int64_t K);
+
+// Row fragments of 64 per tile (2, 3 or 4), or 0 where the fused bodies are the better choice: this path's estimate has
+// to be 7% below the fused body's. This path: expand, rounds of 256 tiles by the measured time of a K step (idle and full
+// chip; more once the expanded matrix leaves the 256 MB cache), the conversion of X. The fused body: its own planner's
+// estimate, scaled, plus the conversion of X and the outputs. Fitted over 14 row counts from 256 to 4096 x 11 shapes, standard
+// deviation 3 to 8% on either side (a flat rate per type misses by up to 35%: fused, Q8_0 4096 x 5120 x 17408 runs at
+// 900 TFLOP/s, 2000 x 17408 x 5120 at 655); of 924 measured calls none that is taken is the slower one, and the choice is within 0.7%
+// of the best one in the mean (up to 15% left: q4_0 3500 x 12288 x 4096, 25600 x 5120 Q5_K at 1400 rows). Measured, fused / here: 17408 x 5120 at 2000 rows q4_0 490 / 489 us (not taken), Q8_0 545 / 474,
+// Q4_K 531 / 472, Q6_K 634 / 476; 5120 x 17408 Q8_0 413 / 474 (not taken), Q6_K 639 / 492; 25600 x 5120 Q8_0 662 / 734 (not taken),
+// at 600 rows Q6_K 307 / 338 (not taken). Calls under 50 us stay fused. At most 2^29 weights (1 GiB of workspace).
 static int wide_plan(int wtype, int64_t M, int64_t N, int64_t K) {
   if (M < 128 || M >= (1 << 24) || K % 256 || K >= (1 << 22) || N % 64 || N * K > (int64_t(1) << 29) || M * K >= (int64_t(1) << 31))
     return 0;
-  double bpw, rate;  // bytes per weight, TFLOP/s of the fused body
+  double bpw, f[4];  // bytes per weight; fused: planner's us, constant, us per 10^6 elements of X and of Y
   switch (wtype) {
-    case 2: bpw = 0.5625, rate = 760; break;
-    case 8: bpw = 1.0625, rate = 700; break;
-    case 12: bpw = 0.5625, rate = 700; break;
-    case 13: bpw = 0.6875, rate = 620; break;
-    case 14: bpw = 0.8203, rate = 460; break;
-    case 22: bpw = 0.3203, rate = 460; break;
+    case 2: bpw = 0.5625, f[0] = 0.511, f[1] = 11.2, f[2] = 0.69, f[3] = 2.86; break;
+    case 8: bpw = 1.0625, f[0] = 0.620, f[1] = 13.8, f[2] = 0.58, f[3] = 2.45; break;
+    case 12: bpw = 0.5625, f[0] = 0.566, f[1] = 12.9, f[2] = 1.02, f[3] = 2.90; break;
+    case 13: bpw = 0.6875, f[0] = 0.661, f[1] = 14.1, f[2] = 0.96, f[3] = 2.76; break;
+    case 14: bpw = 0.8203, f[0] = 0.826, f[1] = 18.4, f[2] = 0.73, f[3] = 0.49; break;
+    case 22: bpw = 0.3203, f[0] = 0.797, f[1] = 16.9, f[2] = 0.43, f[3] = 0.91; break;
     default: return 0;
   }
-  // K step: idle chip, full chip
-  constexpr double step_us[5][2] = {{0, 0}, {0, 0}, {1.0, 1.3}, {1.25, 1.55}, {1.4, 1.8}};
+  const double nk = 1e-6 * static_cast<double>(N) * static_cast<double>(K), mk = 1e-6 * static_cast<double>(M) * static_cast<double>(K);
+  struct Cost {  // us per MB expanded; per K step and round; per K step and full chip, out of cache; per round; constant; per 10^6 of X
+    double exp, step, full, cold, round, fixed, x;
+  };
+  constexpr Cost cost[3] = {{0.148, 0.738, 0.325, 0.283, 10.8, 14.5, 0.06}, {0.123, 1.032, 0.342, 0.206, 18.6, 13.9, 0.17},
+                            {0.151, 1.238, 0.317, 0.168, 31.9, 7.1, 0.38}};
+  const int64_t cus = device_cu_count();
   int best = 0;
   double best_t = -1;
   for (int mf = 2; mf <= 4; ++mf) {
+    const Cost &c = cost[mf - 2];
     const int64_t units = (M + 64 * mf - 1) / (64 * mf) * ((N + 255) / 256);
-    const double rounds = static_cast<double>((units + 255) / 256), use = static_cast<double>(units) / (256 * rounds);
-    const double t = rounds * static_cast<double>(K / 64) * (step_us[mf][0] + use * (step_us[mf][1] - step_us[mf][0])) + 5 * rounds;
+    const double rounds = static_cast<double>((units + cus - 1) / cus), full = static_cast<double>(units) / static_cast<double>(cus);
+    const double t = nk * (2 + bpw) * c.exp + static_cast<double>(K / 64) * (rounds * c.step + full * (c.full + (nk > 120 ? c.cold : 0))) +
+                     rounds * c.round + c.fixed + c.x * mk;
     if (best_t < 0 || t < best_t) best_t = t, best = mf;
   }
   if (const char *e = tuning_env("VYBDQ_WIDE")) {  // 0: never, 2..4: that tile height
-    const int f = atoi(e);
-    return f >= 2 && f <= 4 ? f : 0;
+    const int h = atoi(e);
+    return h >= 2 && h <= 4 ? h : 0;
   }
-  const double nk = static_cast<double>(N) * static_cast<double>(K);
-  return nk * (2 + bpw) / 5.0e6 + best_t + 10 < 0.92 * 2.0 * static_cast<double>(M) * nk / rate / 1e6 ? best : 0;
+  const double fused = f[0] * (wtype >= 14 ? kq2_plan_us(M, N, K) : mmq_plan_us(wtype, M, N, K)) + f[1] + f[2] * mk +
+                       f[3] * 1e-6 * static_cast<double>(M) * static_cast<double>(N);
+  return fused > 50 && best_t < (fused > 500 ? 0.98 : 0.93) * fused ? best : 0;
 }
 
 // workspace: [fp16 weights][fp16 copy of X][X row scales]
-int64_t wide_mm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
-  if (!wide_plan(wtype, M, N, K)) return 0;
+static int64_t wide_bytes(int64_t M, int64_t N, int64_t K) {
   return wide_align256(N * K * 2) + wide_align256(M * K * 2) + wide_align256(M * 4);
+}
+
+int64_t wide_mm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
+  return wide_plan(wtype, M, N, K) ? wide_bytes(M, N, K) : 0;
 }
 
 int x_rows_to_f16(const void *X, int xdt, int64_t M, int64_t K, void *xh, float *xscale, hipStream_t s);
@@ -286,8 +302,9 @@ static int wide_launch(WideArgs &a, hipStream_t s) {
 // Returns 1 when the call does not take this path (rule, or no workspace of wide_mm_workspace_size bytes).
 int wide_mm_gemm(int wtype, const void *W, const void *X, int xdt, void *Y, int ydt, int64_t M, int64_t N, int64_t K,
                  int64_t ldy, const void *RS, void *ws, int64_t ws_bytes, hipStream_t s) {
+  if (!ws || ws_bytes < wide_bytes(M, N, K)) return 1;
   const int mf = wide_plan(wtype, M, N, K);
-  if (!mf || !ws || ws_bytes < wide_mm_workspace_size(wtype, M, N, K)) return 1;
+  if (!mf) return 1;
   char *base = static_cast<char *>(ws);
   char *xh = base + wide_align256(N * K * 2);
   float *sc = reinterpret_cast<float *>(xh + wide_align256(M * K * 2));
