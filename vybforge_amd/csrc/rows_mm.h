@@ -20,8 +20,8 @@
 // sub-blocks' 6-bit mins against their sums of x, split into three fp16 terms. So the weights of these
 // types are not rounded at all. q4_0 / Q8_0 have a scale per 32: their operands are d q, one fp16 product.
 //
-// Measured with the reduce launch, 24 rows bf16, 17408 x 5120 and 5120 x 17408: Q4_K 25.3 and 26.2 us (65 and 136 on the
-// 64-row tiles of kqgemm.hip), Q6_K 32.6 and 34.1 (72 and 177), q4_0 23.3 and 24.1 (47 and 86). The loop
+// Measured with the reduce launch, 24 rows bf16, 17408 x 5120 and 5120 x 17408: Q4_K 26.1 and 26.5 us (65 and 136 on the
+// 64-row tiles of kqgemm.hip), Q6_K 32.6 and 33.4 (72 and 177), q4_0 23.6 and 24.0 (47 and 86). The loop
 // itself streams weights at 4.6 TB/s; the rest is the start (X), the last round of tiles and the
 // reduce (~5 us). Non-finite activations give what the sum over k gives: where the mins are subtracted apart from the
 // products (Q4_K, Q5_K), an infinity would meet zeros and infinities that the weight itself is not, so a row's

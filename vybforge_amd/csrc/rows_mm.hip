@@ -37,12 +37,14 @@ struct RowsPlan {
   int NW, splits, sps, nwg, ns, MF, groups;
 };
 
-// 16 waves (256 weight rows a tile) up to 32 X rows: with 8 (two per SIMD) a wave's decode waits on its
-// own LDS reads and matrix-core chains (Q4_K 17408 x 5120, 24 rows: 25.2 us against 26.9). Above, the accumulators
-// need the registers of 8 waves; and so may LDS (Q8_0: two stages of 256 rows and one X super-block are all
-// of it). One workgroup fits a CU; the plan minimises the stages of the busiest CU (a stage's bytes at
-// the 18.5 GB/s a CU gets of HBM) plus a workgroup's start (X staging) and the split partials, written
-// and read back. With only two LDS stages a stage is barely in flight: 10% more.
+// One workgroup fits a CU; the plan minimises the stages of the busiest CU (a stage's bytes at the 18.5 GB/s a CU gets of HBM)
+// plus a workgroup's start (X staging) and the split partials, written and read back. Up to 32 X rows it has 16 waves (256
+// weight rows a tile) or 8: with 8 (two per SIMD) a wave's decode waits on its own LDS reads and matrix-core chains, 8%; with 16
+// a K range that leaves LDS two stages has one barely in flight, 10% (but not Q6_K, whose decode hides it). Forced, 8 / 16 waves,
+// 17408 x 5120 at 8 rows: q4_0 20.7 / 20.4 us, Q8_0 24.9 / 27.0, Q4_K 21.3 / 20.0, Q5_K 23.5 / 22.3, Q6_K 29.3 / 25.7, IQ2_S 27.7 / 25.2;
+// at 24 rows 24.5 / 23.7, 29.7 / 37.3, 25.9 / 25.0, 28.0 / 27.5, 32.7 / 32.6, 34.7 / 31.8; 4096 x 4096 at 24 rows Q4_K 12.7 / 13.6, Q6_K
+// 13.7 / 14.6; 34816 x 5120 Q4_K 42.4 / 38.6. Over 660 such calls the choice is 0.4% off the better one in the mean, 10% at the
+// worst (8 waves for Q4_K there). Above 32 rows the accumulators need the registers of 8 waves.
 // Up to 2^22 weights the chip is idle and a workgroup's own chain counts, which grows with its X rows (LDS reads of the
 // operands, staging): every 16 rows get workgroups of their own (W again from L2), of 8 waves (twice the workgroups of 16), and a
 // stage costs its latency.
@@ -84,7 +86,7 @@ static RowsPlan rows_plan(int M, int64_t N, int64_t K, int64_t ws_bytes) {
           t = rounds * stages * (FMT == FMT_Q6_K || FMT == FMT_IQ2_S ? 1.85 : 1.2) + static_cast<double>(wgs) / cus;
           if (splits > 1) t += 2.0 + 1.5 * part;
         } else {
-          t = rounds * (stages * stage / 18.5e3 * (ns == 2 ? 1.1 : 1.0) + 2.5 + 0.2 * sps * MF);
+          t = rounds * (stages * stage / 18.5e3 * (ns == 2 && FMT != FMT_Q6_K ? 1.1 : 1.0) + 2.5 + 0.2 * sps * MF);
           if (NW < 16 && MF <= 2) t *= 1.08;
           if (splits > 1) t += 4.0 + 2.0 * part;
         }
