@@ -52,7 +52,7 @@ def test_wide_gemm_residual_ldy(dev, monkeypatch, ydt):
 
 def test_wide_gemm_rule(dev):
     """The rule: a long prompt of a large matrix expands it, a short one does not, and a workspace sized for the
-    fused body still serves the long one."""
+    fused body, or capped below the expanded matrix, still serves the long one."""
     M, N, K = 1024, 9728, 2560
     ty = ops.GGML_Q6_K
     assert ops.GemmWorkspace([(M, N, K)], "cpu", ty).nbytes >= 2 * N * K
@@ -62,6 +62,8 @@ def test_wide_gemm_rule(dev):
     x = torch.from_numpy(synth.activations(rng, (M, K))).to(torch.bfloat16)
     ref = matmul.gemm_rows_f64(x[::97].to(torch.float64).numpy(), w)
     Wd, Xd = to_dev(raw, dev), x.to(dev)
-    for ws in (ops.GemmWorkspace([(M, N, K)], dev, ty), ops.GemmWorkspace([(160, N, K)], dev, ty)):
+    capped = ops.GemmWorkspace([(M, N, K)], dev, ty, max_bytes=2 * N * K)
+    assert capped.nbytes == 2 * N * K
+    for ws in (ops.GemmWorkspace([(M, N, K)], dev, ty), ops.GemmWorkspace([(160, N, K)], dev, ty), capped):
         y = ops.gemm(ty, Wd, Xd, N, K, workspace=ws).cpu().numpy()
         assert matmul.rel_maxnorm(y[::97], ref) < matmul.TOL

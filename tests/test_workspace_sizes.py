@@ -2,7 +2,7 @@
 
 import pytest
 
-from vybforge_amd import _lib
+from vybforge_amd import _lib, ops
 
 ALL = [2, 8, 12, 13, 14, 22]
 
@@ -84,3 +84,12 @@ def test_wide_gemm_is_taken_where_it_measured_faster(ty, M, N, K, wide):
     """Prompts whose matrix is expanded name 2 N K bytes: the shapes on either side of the rule, as measured (the first six
     ran 4 to 12% slower expanded)."""
     assert (gemm_size(ty, M, N, K) >= 2 * N * K + 2 * M * K) == wide
+
+
+def test_gemm_workspace_cap():
+    """A workspace of a long prompt can be capped at what the fused body uses."""
+    M, N, K = 1999, 5120, 17408
+    assert ops.GemmWorkspace([(M, N, K)], "cpu", 14).nbytes >= 2 * N * K
+    ws = ops.GemmWorkspace([(M, N, K)], "cpu", 14, max_bytes=100 << 20)
+    assert ws.nbytes == 100 << 20 and ws.buf.numel() == ws.nbytes + 256
+    assert ops.GemmWorkspace([(1, 64, 256)], "cpu", 14, max_bytes=100 << 20).nbytes == gemm_size(14, 1, 64, 256)

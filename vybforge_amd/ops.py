@@ -421,14 +421,18 @@ def gemm_q8_0_i8(W, Xq, Xs, N, K, y_dtype=torch.float32, residual=None, out=None
 
 class GemmWorkspace:
     """256-byte aligned workspace for vybdq_gemm_ws (int8=False) or vybdq_gemm_q8_0_i8 (int8=True),
-    sized for the given (M, N, K) shapes."""
+    sized for the given (M, N, K) shapes and, up to 64 rows, for every smaller M. Long prompts of large matrices name
+    2 N K bytes more than the fused bodies use (up to 1 GiB, the fp16 weights); max_bytes caps the size, and calls whose
+    path does not fit what is there take the next one that does."""
 
-    def __init__(self, shapes, device, ty=GGML_Q8_0, int8=False):
+    def __init__(self, shapes, device, ty=GGML_Q8_0, int8=False, max_bytes=None):
         if int8:
             sizes = [_lib.lib.vybdq_gemm_q8_0_i8_workspace_size(M, N, K) for M, N, K in shapes]
         else:
             sizes = [_lib.lib.vybdq_gemm_workspace_size(ty, M, N, K) for M, N, K in shapes]
         self.nbytes = max(sizes + [0])
+        if max_bytes is not None:
+            self.nbytes = min(self.nbytes, max_bytes)
         self.buf = torch.zeros(self.nbytes + 256, dtype=torch.uint8, device=device)
         self.ptr = (self.buf.data_ptr() + 255) // 256 * 256 if self.nbytes else 0
 
