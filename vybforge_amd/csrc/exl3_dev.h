@@ -118,7 +118,8 @@ __device__ __forceinline__ void chunk_window(const u4 c, uint32_t (&w)[6]) {
 // whole B operand of v_mfma_f32_16x16x32_f16 (k' = 8 group + 2 row + half). So nothing is
 // regrouped through LDS and nothing is added or packed on the VALU: the matrix core adds x lo + x hi in
 // float32. Shifts s and s + 16 are the two halves of one funnel shift, so eight windows take three
-// of them. VALU instructions per weight: 2 hash products, 1 mask and xor, 3/8 windows = 3.4.
+// of them. Instructions per weight: 2 hash products, 1 mask and xor, 3/8 windows = 3.4 for the decode; 4.0 with the
+// neighbours' dwords, the operands of x and the matrix instructions (8 per 32 weights of a lane).
 
 // the eight windows of dword d (predecessor p), hashed up to their fp16 halves: a = column j, b = column j + 8
 __device__ __forceinline__ void dword_halves(uint32_t p, uint32_t d, u4 &a, u4 &b) {
@@ -148,10 +149,13 @@ __device__ __forceinline__ void exl3_barrier() {
 // step whole 1 KB runs. `base`: the first step's first tile (wave-uniform); `kstride`: uint16 from
 // one k-block to the next; aload(st, v): step st's 16 x' values (k-block l >> 4 of the step) of row
 // l & 15 (any finite or other values for rows past the group: they reach only outputs that are not
-// stored), a step ahead if AHEAD (x' in memory) or at the step (x' in LDS); ready() runs between the first trellis loads and the first aload (it may stage x' in LDS and
-// wait for it: the trellis loads stay in flight across an exl3_barrier). acc[2 c + h][r] = z[row 4 (l >> 4) + r][exl3_mma_col(c, h, l)]. A step of loads (4 KB per
-// wave) is in flight per lane; each ring slot is refilled right after its use, pinned by scheduling
-// barriers (sunk to the end of the step it would leave no load in flight).
+// stored), a step ahead if AHEAD (x' in memory) or at the step (x' in LDS); ready() runs between the
+// first trellis loads and the first aload (it may stage x' in LDS and wait for it: the trellis loads
+// stay in flight across an exl3_barrier). acc[2 c + h][r] = z[row 4 (l >> 4) + r][exl3_mma_col(c, h, l)].
+// A step of loads (4 KB per wave) is in flight per lane; each slot is refilled right after its use,
+// pinned by scheduling barriers (sunk to the end of the step it would leave no load in flight). Two steps in flight
+// (114 VGPRs, four waves per SIMD) measured 3% slower, both where this form has five waves per SIMD (up to 8 rows) and where
+// the partials of 16 rows (33 KB of LDS) leave four workgroups per CU, one wave of each per SIMD.
 template <bool AHEAD, class Ready, class ALoad>
 __device__ __forceinline__ void exl3_mma_run(const uint16_t *__restrict__ base, int64_t kstride, int nsteps,
                                              const Ready &ready, const ALoad &aload, f4 (&acc)[8]) {
@@ -161,7 +165,8 @@ __device__ __forceinline__ void exl3_mma_run(const uint16_t *__restrict__ base, 
   }
   const int lane = threadIdx.x & 63, n = lane & 15;
   const uint16_t *lp = base + (lane >> 4) * kstride + 8 * n;
-  constexpr int R = 1;  // two steps ahead (114 VGPRs, four waves per SIMD instead of five) measured 3% slower
+  // Steps in flight. (A loop over steps alone is the same program, but the compiler then peels the last one: 0.5 to 1.8% slower.)
+  constexpr int R = 1;
   u4 ring[R][4], xr[AHEAD ? R : 1][2];
   auto wload = [&](int st, int c) {
     const int sc = st < nsteps ? st : nsteps - 1;  // in range: re-read the last
@@ -209,7 +214,6 @@ __device__ __forceinline__ void exl3_mma_run(const uint16_t *__restrict__ base, 
 #pragma unroll
     for (int d = 0; d < R; ++d) step(st + d, ring[d], xr[AHEAD ? d : 0]);
   }
-  if (st < nsteps) step(st, ring[0], xr[0]);
 }
 
 // column (of the 128) of accumulator 2 c + h in lane l

@@ -718,7 +718,7 @@ static MxWs mx_layout(char *base, const MxPlan &p, int64_t T, int64_t H, int64_t
 
 template <int SH>
 static int mx_gemm_launch(const MxGemmArgs &a, const MxShared &sh, int nproj, int S, int max_groups, hipStream_t s) {
-  const size_t lds = static_cast<size_t>(4) * a.red_rows * kExl3RedStride * 4;  // 33 KB at 16 rows
+  const size_t lds = static_cast<size_t>(4) * a.red_rows * kExl3RedStride * 4;  // 33 KB at 16 rows: four workgroups per CU
   const unsigned gx = static_cast<unsigned>(max_groups), gz = static_cast<unsigned>(S);
   const unsigned extra = SH ? static_cast<unsigned>((sh.tiles + gx * gz - 1) / (gx * gz)) : 0u;
   MxGemmArgs b = a;
