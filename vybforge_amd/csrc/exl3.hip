@@ -338,12 +338,13 @@ static Exl3Split exl3_splits(int64_t K, int64_t N, int BP) {
     kbs = kbs > 8 ? (kbs + 15) / 16 * 16 : 8;
     return Exl3Split{(KB + kbs - 1) / kbs, kbs};
   };
+  const int64_t cus = device_cu_count();
   Exl3Split best = shape(1);
   int64_t best_cost = -1;
   for (int S = 1; S <= 16; ++S) {
     const Exl3Split c = shape(S);
     if (exl3_lds_bytes(BP, c.kbs) > kExl3MaxLds) continue;
-    const int64_t rounds = (groups * c.S + 255) / 256, steps = 8 * (c.kbs > 16 ? c.kbs : 16);
+    const int64_t rounds = (groups * c.S + cus - 1) / cus, steps = 8 * (c.kbs > 16 ? c.kbs : 16);
     const int64_t cost = exl3_fused(BP) ? rounds * (steps + 8) + 3 * BP * c.kbs + 32 * c.S : rounds * (8 * c.kbs + 48) + 8 * c.S;
     if (best_cost < 0 || cost < best_cost) best_cost = cost, best = c;
   }

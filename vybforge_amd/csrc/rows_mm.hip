@@ -57,7 +57,7 @@ struct RowsPlan {
 template <int FMT>
 static RowsPlan rows_plan(int M, int64_t N, int64_t K, int64_t ws_bytes) {
   using F = RowsFmt<FMT>;
-  const int SB = static_cast<int>(K / 256), MT = (M + 15) / 16, cus = 256, tab = FMT == FMT_IQ2_S ? kRowsGrid : 0;
+  const int SB = static_cast<int>(K / 256), MT = (M + 15) / 16, cus = device_cu_count(), tab = FMT == FMT_IQ2_S ? kRowsGrid : 0;
   RowsPlan best{};
   double best_t = -1;
   int fs = 0, fn = 0, fg = 0;
