@@ -93,12 +93,13 @@ def test_exl3_gemm_config4_shape(dev, exl3_config4, B, xdt):
         assert matmul.rel_maxnorm(y[:, c0:c0 + 1024], ref) < matmul.TOL, (B, c0)
 
 
-@pytest.mark.parametrize("K,N", [(128, 256), (1152, 256), (2048, 384)])
+@pytest.mark.parametrize("K,N", [(128, 256), (1152, 256), (2048, 384), (4224, 256)])
 def test_exl3_gemm_splits_and_reuse(dev, K, N):
     """One workspace across calls of several batch sizes and dtypes (the per-block arrival
     counters must come back to zero after every call): a single k-split of two 64-k steps (K = 128:
-    two of the four waves idle), a ragged last split (K = 1152: four splits of 256 k and one of
-    128), even splits (K = 2048), repeated calls bit-identical."""
+    two of the four waves idle), a ragged last split at batch <= 2 (K = 1152: four splits of 256 k and
+    one of 128; nine of 128 above) and at every batch (K = 4224: eight of 512 and one of 128), even splits
+    (K = 2048), repeated calls bit-identical."""
     rng = np.random.default_rng(K + N)
     t, suh, svh = synth.exl3_tensors(rng, K, N)
     lin = ops.Exl3Linear(dev_t(t, dev), dev_t(suh, dev), dev_t(svh, dev), K, N)
