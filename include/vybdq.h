@@ -299,7 +299,7 @@ int vybdq_exl3_decode_tiles(uint64_t trellis, uint64_t out, int64_t K, int64_t N
 int vybdq_dequant_exl3(uint64_t trellis, uint64_t suh, uint64_t svh, uint64_t out, int64_t K, int64_t N,
                        int codebook, int out_dt, uint64_t stream);
 
-/* Workspace bytes for vybdq_exl3_gemm at (B, K, N), or -1 for an unsupported shape. */
+/* Workspace bytes for vybdq_exl3_gemm at (B, K, N) and every smaller batch, or -1 for an unsupported shape. */
 int64_t vybdq_exl3_workspace_size(int64_t B, int64_t K, int64_t N);
 
 /* Y [B, N] = X [B, K] W, W the EXL3 matrix above, without materialising W: X is rotated
@@ -338,9 +338,9 @@ int vybdq_gemm(int wtype, uint64_t W, uint64_t X, uint64_t Y, int64_t M, int64_t
                int y_dt, int64_t ldy, uint64_t RS, uint64_t stream);
 
 /* Workspace bytes vybdq_gemm_ws can use at (M, N, K) (up to 64 rows, K % 256 == 0, N % 64 == 0: split-K
-   partials; q4_0, Q8_0, Q4_K, Q5_K from 64 rows, Q6_K, IQ2_S from 96 rows: split-K partials and the
-   fp16 copy of a bf16/f32 X; long prompts of large matrices: 2 N K bytes more, the fp16 weights); 0 when
-   the shape does not use the workspace. */
+   partials, of M rows or any smaller count; q4_0, Q8_0, Q4_K, Q5_K from 64 rows, Q6_K, IQ2_S from 96 rows: split-K
+   partials and the fp16 copy of a bf16/f32 X, and what 64 rows use; long prompts of large matrices: 2 N K bytes for the
+   fp16 weights besides X); 0 when the shape does not use the workspace. */
 int64_t vybdq_gemm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
 
 /* vybdq_gemm with a caller workspace ws (256-byte aligned, ws_bytes, any contents; 0 = none). With
@@ -351,8 +351,10 @@ int64_t vybdq_gemm_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
    once per output tile, each row scaled by the power of two that brings its largest |x| into
    [2^14, 2^15) (multiplied back into the row's outputs), so X of any magnitude neither overflows nor
    flushes to zero. Up to 64 rows (K % 256 == 0, N % 64 == 0, W 16-byte aligned) the call runs on weights
-   streamed past X in LDS, X scaled the same way per row and 256 k; Q4_K, Q5_K, Q6_K and IQ2_S weights
-   are not rounded to fp16 there. Long prompts of large matrices (the size tells: 2 N K bytes more) expand
+   streamed past X in LDS, X scaled the same way per row and 256 k, in as many K splits as the workspace
+   has room for (too small for any: as without one); Q4_K, Q5_K and IQ2_S weights are not rounded to fp16 there, and
+   of Q6_K only those whose scale times quant passes 2048; infinities and NaNs of X give what the sum over k gives.
+   Long prompts of large matrices (the size tells: 2 N K bytes) expand
    W to fp16 in the workspace once and run a plain fp16 tile GEMM over it; a smaller workspace keeps the
    fused bodies. Calls that share a workspace must not overlap. The reference's gemm_q80
    has no workspace (native/tools/gen_rpf.py:58-62); this is the same GEMM for shapes whose
@@ -506,7 +508,7 @@ int vybdq_moe_forward_noalloc(int wtype, uint64_t x, int x_dt, uint64_t logits, 
 
 /* ---- MoE layer with EXL3 routed experts -------------------------------------------------- */
 
-/* Workspace bytes for vybdq_moe_forward_exl3, or -1 for an unsupported shape. */
+/* Workspace bytes for vybdq_moe_forward_exl3 with T or fewer tokens, or -1 for an unsupported shape. */
 int64_t vybdq_moe_exl3_workspace_size(int64_t T, int64_t H, int64_t I, int64_t E, int64_t topk);
 
 /* The reference's production GLM-5.3 MoE layer (native/glm53/glm_engine.vyb:2728-2990) in one call:
