@@ -187,3 +187,22 @@ def test_rows_gemm_non_finite(dev, ty, xdt, M, N, K):
     assert not np.isfinite(y[bad]).any()
     good = [m for m in range(M) if m not in bad]
     assert matmul.rel_maxnorm(y[good], ref[good]) < matmul.TOL
+
+
+@pytest.mark.parametrize("ty", TYPES)
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+def test_gemm_one_workspace_above_64_rows(dev, ty, xdt):
+    """A workspace sized for 257 rows of a short matrix holds less than the K splits of 129 rows and their scaled copy
+    of X: the copy is kept, and activations of any magnitude match at every smaller count."""
+    N, K, Mmax = 192, 1024, 257
+    rng = np.random.default_rng(ty)
+    raw, w = weights(ty, rng, N, K)
+    xd, x64 = x_as(_x_pattern("huge", rng, Mmax, K), xdt, dev)
+    Wd, x64 = to_dev(raw, dev), x64.reshape(Mmax, K)
+    ws = ops.GemmWorkspace([(Mmax, N, K)], dev, ty)
+    ref = matmul.gemm_rows_f64(x64, w)
+    for M in (65, 96, 128, 129, 200, 256, 257):
+        if M < 96 and ty in (ops.GGML_Q6_K, ops.GGML_IQ2_S):
+            continue  # the 64-row tiles, which take X as it is
+        y = ops.gemm(ty, Wd, xd.reshape(Mmax, K)[:M], N, K, workspace=ws).cpu().numpy()
+        assert np.all(np.isfinite(y)) and matmul.rel_maxnorm(y, ref[:M]) < matmul.TOL, M

@@ -35,6 +35,7 @@ enum { EPI_STORE = 0, EPI_SWIGLU = 1 };
 // the MFMA GEMM with weights in operand registers (mmq_host.hip)
 bool mmq_supported(int64_t M, int64_t N, int64_t K);
 int64_t mmq_workspace_size(int wtype, int64_t M, int64_t N, int64_t K);
+int64_t mmq_x_bytes(int64_t M, int64_t K);
 int mmq_gemm(int wtype, const void *W, const void *X, int xdt, void *Y, int ydt, int64_t M, int64_t N, int64_t K,
              int64_t ldy, const void *RS, void *ws, int64_t ws_bytes, hipStream_t s);
 int64_t mmq_i8_workspace_size(int64_t M, int64_t N, int64_t K);
@@ -499,7 +500,7 @@ extern "C" int vybdq_gemm_ws(int wtype, uint64_t W, uint64_t X, uint64_t Y, int6
   // Q4_K / Q5_K: the register-operand body streams fp16 X, so bf16 / f32 X needs room for its
   // conversion
   const bool q4k_ok = (wtype == 12 || wtype == 13) && M >= 64 && K < (int64_t(1) << 22) && mmq_supported(M, N, K) &&
-                      (x_dt == VYBDQ_F16 || (ws && ws_bytes >= mmq_workspace_size(wtype, M, N, K)));
+                      (x_dt == VYBDQ_F16 || (ws && ws_bytes >= mmq_x_bytes(M, K)));
   if (wtype == 14 || wtype == 22) {  // 128-row tiles over the workspace's fp16 copy of X
     const int r = kq2_gemm(wtype, reinterpret_cast<const void *>(W), reinterpret_cast<const void *>(X), x_dt,
                            reinterpret_cast<void *>(Y), y_dt, M, N, K, ldy ? ldy : N,

@@ -143,12 +143,18 @@ int64_t mmq_workspace_size(int wtype, int64_t M, int64_t N, int64_t K) {
          align256(M * K * 2) + align256(M * 4);
 }
 
+// room for the scaled fp16 copy of X alone
+int64_t mmq_x_bytes(int64_t M, int64_t K) { return align256(M * K * 2) + M * 4; }
+
 int mmq_gemm(int wtype, const void *W, const void *X, int xdt, void *Y, int ydt, int64_t M, int64_t N, int64_t K,
              int64_t ldy, const void *RS, void *ws, int64_t ws_bytes, hipStream_t s) {
   const int S = static_cast<int>(K / 128);
   MmPlan p = mm_plan(static_cast<int>(M), static_cast<int>(N), S, ws != nullptr, mm_nfx(wtype));
-  if (p.splits > 1 && ws_bytes < p.ws_bytes) p = mm_plan(static_cast<int>(M), static_cast<int>(N), S, false, mm_nfx(wtype));
-  // with room for it, a non-fp16 X is converted once up front (instead of once per N tile)
+  // with room for it, a non-fp16 X is converted once up front (instead of once per N tile); a workspace that holds the
+  // scaled copy but not the partials beside it keeps the copy and leaves K whole
+  const int64_t xbytes = xdt != VYBDQ_F16 ? mmq_x_bytes(M, K) : 0;
+  if (p.splits > 1 && (ws_bytes < p.ws_bytes || (ws_bytes >= xbytes && ws_bytes < align256(p.ws_bytes) + xbytes)))
+    p = mm_plan(static_cast<int>(M), static_cast<int>(N), S, false, mm_nfx(wtype));
   const int64_t xh_off = align256(p.ws_bytes);
   const int64_t sc_off = xh_off + align256(M * K * 2);
   const float *xscale = nullptr;
