@@ -190,6 +190,38 @@ def test_rows_gemm_non_finite(dev, ty, xdt, M, N, K):
 
 
 @pytest.mark.parametrize("ty", TYPES)
+@pytest.mark.parametrize("M", [3, 20, 37, 50, 63])
+@pytest.mark.parametrize("plan,splits", [("2,2", 1), ("1,3", 2)])
+def test_rows_gemm_non_finite_in_place(dev, ty, M, plan, splits, monkeypatch):
+    """Non-finite rows of X where a workgroup walks several tiles and Y is its own residual with a row stride: the
+    residual is read once, columns past N stay."""
+    monkeypatch.setenv("VYBDQ_TUNING", "1")
+    monkeypatch.setenv("VYBDQ_ROWS_PLAN", plan)
+    N, K, ldy = 896, 512, 1000
+    rng = np.random.default_rng(ty + M)
+    raw, w = weights(ty, rng, N, K)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    x[0, 5] = np.inf
+    x[1, [200, 300]] = -np.inf, np.inf
+    x[M - 1, K - 1] = np.nan
+    rs = synth.activations(rng, (M, ldy)).astype(np.float64)
+    Wd, Xd, y = to_dev(raw, dev), to_dev(x, dev), to_dev(rs, dev)
+    ws = ops.GemmWorkspace([(M, N, K)], dev, ty)
+    assert ws.nbytes == (splits * M * N * 4 if splits > 1 else 256)  # the forced plan
+    call("vybdq_gemm_ws", ty, Wd.data_ptr(), Xd.data_ptr(), y.data_ptr(), M, N, K, ops.F16, ops._dt(torch.float64), ldy,
+         y.data_ptr(), ws.ptr, ws.nbytes, torch.cuda.current_stream().cuda_stream)
+    got = y.cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        ref = rs[:, :N] + (x.astype(np.float64).reshape(M, 1, K) * np.asarray(w, dtype=np.float64)[None]).sum(-1)
+    bad = [0, 1, M - 1]
+    np.testing.assert_array_equal(got[bad, :N], ref[bad])
+    good = [m for m in range(M) if m not in bad]
+    if good:
+        assert matmul.rel_maxnorm(got[good, :N], ref[good]) < matmul.TOL
+    np.testing.assert_array_equal(got[:, N:], rs[:, N:])
+
+
+@pytest.mark.parametrize("ty", TYPES)
 @pytest.mark.parametrize("xdt", ["bf16", "f32"])
 def test_gemm_one_workspace_above_64_rows(dev, ty, xdt):
     """A workspace sized for 257 rows of a short matrix holds less than the K splits of 129 rows and their scaled copy

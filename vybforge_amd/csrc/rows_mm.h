@@ -25,8 +25,8 @@
 // itself streams weights at 4.6 TB/s; the rest is the start (X), the last round of tiles and the
 // reduce (~5 us). Non-finite activations give what the sum over k gives: where the mins are subtracted apart from the
 // products (Q4_K, Q5_K), an infinity would meet zeros and infinities that the weight itself is not, so a row's
-// super-block that holds one is staged as zeros under an infinite scale, and a tile that then holds NaNs takes those rows'
-// infinities (and NaNs) times whole weights instead.
+// super-block that holds one is staged as zeros under an infinite scale, and where a tile then holds NaNs, those rows are
+// left to the end: their infinities (and NaNs) times whole weights.
 #pragma once
 #include "gemv_dev.h"
 
@@ -173,28 +173,50 @@ typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 
 template <int XDT> struct RowsX { u4 r[XDT == VYBDQ_F32 ? 2 : 1]; };
 
-// The rows of a tile whose super-blocks were marked (scale infinite, operands zero: the accumulators of those rows are
-// NaN): their non-finite activations times whole weights, the other terms being finite. All lanes of the wave; column col,
-// unit g, split super-blocks sb0 .. sb0 + nst.
+// Whether row R of the workgroup has a marked super-block (scale infinite, operands zero) in its K range
+template <int FMT, int MF>
+__device__ __forceinline__ bool rows_marked(const char *xs, int nst, int R) {
+  using F = RowsFmt<FMT>;
+  constexpr int XSB = MF * (F::OPS * 1024 + 64);
+  for (int b = 0; b < nst; ++b)
+    if (!(reinterpret_cast<const float *>(xs + b * XSB + MF * F::OPS * 1024)[R] < __builtin_inff())) return true;
+  return false;
+}
+
+// value of row, col: this K range's partial, or the output
+__device__ __forceinline__ void rows_store(const RowsArgs &a, int row, int64_t col, float v) {
+  if (a.splits > 1) {
+    a.part[(static_cast<int64_t>(blockIdx.y) * a.M + row) * a.N + col] = v;
+    return;
+  }
+  const int64_t i = static_cast<int64_t>(row) * a.ldy + col;
+  switch (a.ydt) {
+    case VYBDQ_F32: store_elem<VYBDQ_F32>(a.Y, a.RS, i, v); break;
+    case VYBDQ_F16: store_elem<VYBDQ_F16>(a.Y, a.RS, i, v); break;
+    case VYBDQ_BF16: store_elem<VYBDQ_BF16>(a.Y, a.RS, i, v); break;
+    default: store_elem<VYBDQ_F64>(a.Y, a.RS, i, v); break;
+  }
+}
+
+// The marked rows of a tile, whose accumulators are NaN: their non-finite activations times whole weights (the other
+// terms are finite), stored. All lanes of the wave; column col, unit g, split super-blocks sb0 .. sb0 + nst.
 template <int FMT, int XDT, int MF>
-__device__ __forceinline__ void rows_non_finite(const RowsArgs &a, const char *xs, int sb0, int nst, int m0, int64_t col, int g,
-                                                f4 (&acc)[MF]) {
+__device__ __forceinline__ void rows_non_finite(const RowsArgs &a, const char *xs, int sb0, int nst, int m0, int64_t col, int g) {
   using F = RowsFmt<FMT>;
   constexpr int XSB = MF * (F::OPS * 1024 + 64);
 #pragma unroll 1
-  for (int R = 0; R < 16 * MF; ++R) {
+  for (int R = 0; R < 16 * MF && m0 + R < a.M; ++R) {
+    if (!rows_marked<FMT, MF>(xs, nst, R)) continue;
     float s = 0.f;
-    bool marked = false;
 #pragma unroll 1
     for (int b = 0; b < nst; ++b) {
       if (reinterpret_cast<const float *>(xs + b * XSB + MF * F::OPS * 1024)[R] < __builtin_inff()) continue;
-      marked = true;
       const uint8_t *sb = a.W + col * a.rowbytes + static_cast<int64_t>(sb0 + b) * F::SBB;
       const uint32_t *hd = reinterpret_cast<const uint32_t *>(sb);
       const float d = half_bits_to_f32(hd[0] & 0xffffu), dmin = half_bits_to_f32(hd[0] >> 16);
       uint32_t sc6, mn6;
       rows_scales_k4(hd[1], hd[2], hd[3], g, sc6, mn6);
-      const int64_t e0 = (min(m0 + R, a.M - 1) * static_cast<int64_t>(a.SB) + sb0 + b) * 256 + 64 * g;
+      const int64_t e0 = ((m0 + R) * static_cast<int64_t>(a.SB) + sb0 + b) * 256 + 64 * g;
 #pragma unroll 1
       for (int i = 0; i < 64; ++i) {
         const float x = load_elem<XDT>(a.X, e0 + i);
@@ -206,13 +228,9 @@ __device__ __forceinline__ void rows_non_finite(const RowsArgs &a, const char *x
                       -dmin * static_cast<float>((mn6 >> (8 * h)) & 0xffu));
       }
     }
-    if (!marked) continue;
     s += __shfl_xor(s, 16, 64);
     s += __shfl_xor(s, 32, 64);
-#pragma unroll
-    for (int m = 0; m < MF; ++m)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[m][r] = R == 16 * m + 4 * g + r ? s : acc[m][r];
+    if (g == 0) rows_store(a, m0 + R, col, s);
   }
 }
 
@@ -403,6 +421,7 @@ __global__ void __launch_bounds__(64 * NW) k_rows_mm(const RowsArgs a) {
   for (int m = 0; m < MF; ++m) acc[m] = f4{0.f, 0.f, 0.f, 0.f};
   const int row0 = wave * 16 + n;  // this lane's weight row within the tile
   int tile = blockIdx.x, sbl = 0, cb = 0;
+  bool fix = false;  // a tile had rows of marked super-blocks
   for (int z = 0; z < total; ++z) {
     wait_later(min(NS - 2, total - 1 - z));
     bar();
@@ -464,36 +483,54 @@ __global__ void __launch_bounds__(64 * NW) k_rows_mm(const RowsArgs a) {
     if (++sbl < nst) continue;
     // acc[m][r] = C[m0 + 16 m + 4 g + r][BN tile + row0]
     const int64_t col = static_cast<int64_t>(tile) * Sh::BN + row0;
+    int lim = a.M;
     if constexpr (F::MINS) {
       bool nan = false;
 #pragma unroll
       for (int m = 0; m < MF; ++m)
 #pragma unroll
         for (int r = 0; r < 4; ++r) nan |= acc[m][r] != acc[m][r];
-      if (__any(nan)) rows_non_finite<FMT, XDT, MF>(a, xs, sb0, nst, m0, col, g, acc);
+      if (__any(nan)) {  // stored here but for the marked rows, which follow the last tile
+        fix = true;
+        lim = 0;
+#pragma unroll 1
+        for (int i = 0; i < 4 * MF; ++i) {
+          float v = 0.f;
+#pragma unroll
+          for (int m = 0; m < MF; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v = i == 4 * m + r ? acc[m][r] : v;
+          const int R = 16 * (i >> 2) + 4 * g + (i & 3);
+          if (m0 + R < a.M && !rows_marked<FMT, MF>(xs, nst, R)) rows_store(a, m0 + R, col, v);
+        }
+      }
     }
 #pragma unroll
     for (int m = 0; m < MF; ++m) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = m0 + 16 * m + 4 * g + r;
-        if (row >= a.M) continue;
-        if (a.splits > 1) {
-          a.part[(static_cast<int64_t>(blockIdx.y) * a.M + row) * a.N + col] = acc[m][r];
-          continue;
-        }
-        const int64_t i = static_cast<int64_t>(row) * a.ldy + col;
-        switch (a.ydt) {
-          case VYBDQ_F32: store_elem<VYBDQ_F32>(a.Y, a.RS, i, acc[m][r]); break;
-          case VYBDQ_F16: store_elem<VYBDQ_F16>(a.Y, a.RS, i, acc[m][r]); break;
-          case VYBDQ_BF16: store_elem<VYBDQ_BF16>(a.Y, a.RS, i, acc[m][r]); break;
-          default: store_elem<VYBDQ_F64>(a.Y, a.RS, i, acc[m][r]); break;
-        }
+        if (row < lim) rows_store(a, row, col, acc[m][r]);
       }
       acc[m] = f4{0.f, 0.f, 0.f, 0.f};
     }
     sbl = 0;
     tile += gridDim.x;
+  }
+  if constexpr (F::MINS) {
+    if (fix) {
+      // Arguments and lane are read again, so that nothing here is computed ahead of the tile loop or kept over it: inside
+      // the loop, with its values shared, this took 5 to 10% of every call of 49 to 64 rows (Q4_K 17408 x 5120, 64 rows
+      // 40.7 us; like this 37.8, without it 37.0).
+      const RowsArgs *ap = (const RowsArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+      int tid = threadIdx.x;
+      char *sm = smem;
+      asm volatile("" : "+s"(ap), "+v"(tid), "+v"(sm));
+      const int s0 = blockIdx.y * ap->sps;
+      for (int t = blockIdx.x; t < ap->tiles; t += gridDim.x)
+        rows_non_finite<FMT, XDT, MF>(*ap, sm + Sh::TAB, s0, min(ap->sps, ap->SB - s0), GR ? blockIdx.z * 16 * MF : 0,
+                                      static_cast<int64_t>(t) * Sh::BN + (tid >> 6) * 16 + (tid & 15), (tid & 63) >> 4);
+    }
   }
 }
 
